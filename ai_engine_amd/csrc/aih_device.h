@@ -6,7 +6,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <mutex>
+#include <atomic>
 
 #include "../../include/aih_conv.h"
 
@@ -294,19 +294,20 @@ struct DeviceInfo {
 };
 
 inline DeviceInfo device_info() {
-  static std::mutex mu;
-  static DeviceInfo cache[64] = {};
+  // one word per device, CUs above XCDs; 0: not asked yet. Threads that ask
+  // at once store the same word.
+  static std::atomic<uint64_t> cache[64] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return DeviceInfo{256, 8};
-  std::lock_guard<std::mutex> lock(mu);
-  DeviceInfo &d = cache[dev];
-  if (d.cus == 0) {
+  uint64_t v = cache[dev].load(std::memory_order_relaxed);
+  if (v == 0) {
     int cus = 0, xcds = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
     if (hipDeviceGetAttribute(&xcds, hipDeviceAttributeNumberOfXccs, dev) != hipSuccess || xcds <= 0) xcds = 8;
-    d = DeviceInfo{(uint32_t)cus, (uint32_t)xcds};
+    v = (uint64_t)cus << 32 | (uint32_t)xcds;
+    cache[dev].store(v, std::memory_order_relaxed);
   }
-  return d;
+  return DeviceInfo{(uint32_t)(v >> 32), (uint32_t)v};
 }
 inline uint32_t device_cus() { return device_info().cus; }
 inline uint32_t device_xcds() { return device_info().xcds; }

@@ -26,6 +26,7 @@
 #include "conv_pw_splitk.h"
 #include "conv_pw_stream.h"
 #include "conv_stem.h"
+#include "conv_stream.h"
 #include "ir_block.h"
 
 std::string &aih::last_error_slot() {
@@ -289,6 +290,44 @@ bool pw_stream_plan(const aih_pw_desc *d, aih::PwStreamArgs *a, aih::PwStreamSha
   return true;
 }
 
+// The LDS-streamed conv GEMM's tile for M pixels x N4 outputs (conv_stream.hip)
+// and the arguments that depend on it. More than 64 outputs: the wide tile
+// that pads the columns least, 64- and 96-column tiles counted at 5/4 of
+// their columns at 16 bit, where the LDS reads per MFMA bound them (320 ->
+// 576 bf16 at 40x72 b64: 128 us at 128 columns, 64 of them padding, 153 at
+// 64, 158 at 96; fp32 3x3 64 -> 128 b32: 117 and 121). Up to 64 outputs, and
+// where the wide tiles are fewer than two per CU: 64 x 64 (3x3 256 -> 256
+// f16 at 40x72 b4: 180 tiles of 128 x 128 41.9 us, 720 of 64 x 64 24.8).
+void conv_stream_tile(aih::ConvStreamArgs *a, int32_t dt, aih::ConvStreamShape *shape) {
+  const aih::ConvStreamShape *best = nullptr;
+  uint64_t best_cost = 0;
+  for (const aih::ConvStreamShape &sh : aih::kConvStreamWide) {
+    const uint64_t bn = aih::conv_stream_bn(sh);
+    const uint64_t cost = div_ceil(a->N4, (uint32_t)bn) * bn * (bn == 128 || dt == AIH_F32 ? 4 : 5);
+    if (!best || cost < best_cost) {
+      best = &sh;
+      best_cost = cost;
+    }
+  }
+  const uint64_t wide = (uint64_t)div_ceil(a->M, aih::conv_stream_bm(*best)) * div_ceil(a->N4, aih::conv_stream_bn(*best));
+  if (a->N4 <= 64 || wide < 2ull * aih::device_cus())
+    // stages of 8 units pay off over a long K (960 -> 24 f16 at 40x72 b64:
+    // 79.7 -> 69.1 us) and cost padding units in a short pointwise one (72 ->
+    // 192: 23.2 -> 29.4); a KxK conv's taps run on without padding
+    best = &aih::kConvStreamSmall[(a->K > 1 ? a->KU >= 8 : a->KU >= 40) ? 0 : 1];
+  const uint32_t mtiles = div_ceil(a->M, aih::conv_stream_bm(*best));
+  const uint32_t ntiles = div_ceil(a->N4, aih::conv_stream_bn(*best));
+  a->mtiles = mtiles;
+  a->ntiles = ntiles;
+  a->nst = div_ceil(a->K * a->K * a->KU, best->bku);
+  a->fd_nt = aih::make_fastdiv(a->ntiles);
+  a->nxcd = aih::device_xcds();
+  *shape = *best;
+}
+
+// Whether the kernel's grid fits a launch.
+bool conv_stream_grid_ok(const aih::ConvStreamArgs &a) { return (uint64_t)a.mtiles * a.ntiles <= 0x7fffffffull; }
+
 // The split factor of a pointwise call: the descriptor's, else (AUTO only)
 // the AIH_PW_SPLITK override, else 0 (the policy decides).
 int32_t pw_splitk_of(const aih_pw_desc *d) {
@@ -309,7 +348,8 @@ bool pw_splitk_waves_ok(int32_t w) {
   return false;
 }
 
-int pw_route(const aih_pw_desc *d) {
+// The route without the LDS-streamed conv GEMM (pw_dma_plan, below).
+int pw_base_route(const aih_pw_desc *d) {
   const int32_t sk = pw_splitk_of(d);
   if (d->variant == AIH_VAR_AUTO && sk > 0)
     // a forced factor: one dispatch with that many K chunks where the shape
@@ -338,6 +378,65 @@ int pw_route(const aih_pw_desc *d) {
       ((M + aih::GEMM_BM - 1) / aih::GEMM_BM) * ((d->ng * 4 + 31) / 32) < aih::device_cus())
     return PW_SPLITK;
   return PW_TILED;
+}
+
+int plan_pw(const aih_pw_desc *d, GemmPlan *g) {
+  return plan_gemm(d->n * d->m, d->ng * 4, d->kg, d->dt, d->variant, pw_splitk_of(d), g);
+}
+
+// A pointwise call of base route `base` on the LDS-streamed conv GEMM
+// (conv_stream.hip): AIH_VAR_AUTO without a forced split, the same storage
+// for activations and weights, whole 16-byte units, at least 4 of them,
+// buffers within 32-bit offsets.
+//   16 bit: what the tiled GEMM ran (192 -> 768 at 21x37 b64: 64.5 -> 35 us),
+//   and what the direct kernels ran with more than 32 outputs or at least 64
+//   channels, beyond 2048 pixels (32 -> 64 at 80x144 b64: 56.7 -> 35 us, 128
+//   -> 32 at 40x72 b64: 19.6 -> 12.6, 128 -> 64 at 11520 pixels 5.9 -> 3.5;
+//   below both, 32 -> 16 at 40x72 b64: 6.0 us there, 7.0 here).
+//   fp32: what the tiled GEMM ran with K whole (128 -> 320 at 20x36 b64: 74
+//   -> 43 us); calls it splits keep the split's shorter sums.
+// need: the workspace the call is checked against, the tiled GEMM's where
+// that is the base route (also for calls that run here without one).
+bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::ConvStreamShape *shape, size_t *need) {
+  *need = 0;
+  const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;
+  if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || d->dt != d->wdt || d->kg % ku || d->kg / ku < 4)
+    return false;
+  const uint64_t M = (uint64_t)d->n * d->m, N4 = (uint64_t)d->ng * 4;
+  const uint64_t xb = M * d->kg * 4 * es, wb = (uint64_t)d->kg_pad * N4 * 4 * es;
+  if (M <= aih::kPwSplitkMaxM || xb >= 0x80000000ull || wb >= 0x80000000ull) return false;
+  if (base == PW_DIRECT || base == PW_LDS || base == PW_SPLITK) {
+    if (d->dt == AIH_F32 || (N4 <= 32 && d->kg < 16)) return false;
+    // 16x16-block launches of a short K stay
+    if (base == PW_SPLITK && d->kg < 16) return false;
+  } else if (base == PW_TILED) {
+    GemmPlan g;
+    if (plan_pw(d, &g) || (d->dt == AIH_F32 && g.nsplit > 1)) return false;
+    *need = g.ws;
+  } else {
+    return false;
+  }
+  std::memset(a, 0, sizeof(*a));
+  a->x_bytes = (uint32_t)xb;
+  a->w_bytes = (uint32_t)wb;
+  a->M = (uint32_t)M;
+  a->KU = a->stride_u = d->kg / ku;
+  a->KG = d->kg;
+  a->KGP = d->kg_pad;
+  a->N4 = (uint32_t)N4;
+  a->OHW = a->OW = a->IW = d->m;
+  a->IH = a->K = a->S = a->D = 1;
+  a->fd_ohw = a->fd_ow = aih::make_fastdiv(d->m);
+  a->act = d->act;
+  a->has_res = d->residual ? 1 : 0;
+  conv_stream_tile(a, d->dt, shape);
+  return conv_stream_grid_ok(*a);
+}
+
+// The workspace of a pointwise call of base route `base`.
+size_t pw_ws(const aih_pw_desc *d, int base) {
+  GemmPlan g;
+  return base == PW_TILED && !plan_pw(d, &g) ? g.ws : 0;
 }
 
 // Arguments of the one-dispatch split-K kernel and its K chunks (waves).
@@ -406,10 +505,6 @@ int check_pw(const aih_pw_desc *d) {
   if ((uint64_t)d->n * d->m > 0xffffffffull / 4) return fail("pw: too many pixels");
   if ((uint64_t)d->n * d->m * d->kg > 0xffffffffull) return fail("pw: input too large");
   return AIH_OK;
-}
-
-int plan_pw(const aih_pw_desc *d, GemmPlan *g) {
-  return plan_gemm(d->n * d->m, d->ng * 4, d->kg, d->dt, d->variant, pw_splitk_of(d), g);
 }
 
 // ---------------------------------------------------------------- igemm
@@ -548,6 +643,64 @@ bool ig_direct_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::IgDi
   a->fd_ohw = aih::make_fastdiv(oh * ow);
   a->fd_ow = aih::make_fastdiv(ow);
   return true;
+}
+
+// A KxK call on the LDS-streamed conv GEMM: AIH_VAR_AUTO without a forced
+// split, the same storage for activations and weights, one input (plain or a
+// channel view) whose kg count, pixel stride and offset are whole 16-byte
+// units, at least 4 units a tap, buffers within 32-bit offsets. direct: the
+// call is one of the direct 3x3 kernel's; unsplit: the tiled GEMM keeps K
+// whole.
+//   tiled calls at 16 bit: from 48 tiles of 64 x 64 (128 -> 128 3x3 at 40x72
+//   b32: 69.7 -> 41 us; fewer tiles, 256 -> 256 at 10x18 b4 is 48 of them:
+//   18.1 -> 15.8); at fp32 the unsplit ones (64 -> 128 b32: 222 -> 117 us;
+//   split ones keep the split's shorter sums).
+//   direct calls below 65536 pixels, whose 32-pixel wavefronts leave CUs idle
+//   (64 -> 64 fp32 at 40x72 b4: 44 -> 17 us, f16 15.3 -> 6.6); at fp32 only
+//   with more than 32 outputs (72 -> 32 b8: 29.7 there, 30.1 here); at or
+//   above, 16-bit ones with whole 64-channel taps (64 -> 64 b32: 22.4 -> 17.8,
+//   128 -> 64 38.2 -> 28.8; 96 -> 64 22.6 there, 25.5 here).
+bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool direct, bool unsplit,
+                       aih::ConvStreamArgs *a, aih::ConvStreamShape *shape) {
+  if (d->variant != AIH_VAR_AUTO || d->splitk != 0 || d->dt != d->wdt || d->nsrcs > 1) return false;
+  const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;
+  const uint32_t kg = div_ceil(d->cin, 4), n4 = div_ceil(d->cout, 4) * 4;
+  const uint32_t stride = d->nsrcs ? d->srcs[0].stride_c / 4 : kg, off = d->nsrcs ? d->srcs[0].c_off / 4 : 0;
+  if (kg % ku || stride % ku || off % ku || kg / ku < 4) return false;
+  const uint32_t M = d->n * oh * ow;
+  if (direct) {
+    if (M < 65536 ? d->dt == AIH_F32 && n4 <= 32 : d->dt == AIH_F32 || kg % 16) return false;
+  } else {
+    if (d->dt == AIH_F32 ? !unsplit : (uint64_t)div_ceil(M, 64) * div_ceil(n4, 64) < 48) return false;
+  }
+  const uint32_t kgp = div_ceil(kg, 4) * 4;
+  const uint64_t xb = (uint64_t)d->n * d->ih * d->iw * stride * 4 * es, wb = (uint64_t)d->k * d->k * kgp * n4 * 4 * es;
+  if (xb >= 0x80000000ull || wb >= 0x80000000ull) return false;
+  std::memset(a, 0, sizeof(*a));
+  a->x_bytes = (uint32_t)xb;
+  a->w_bytes = (uint32_t)wb;
+  a->M = M;
+  a->KU = kg / ku;
+  a->KG = kg;
+  a->KGP = kgp;
+  a->stride_u = stride / ku;
+  a->off_u = off / ku;
+  a->N4 = n4;
+  a->OHW = oh * ow;
+  a->OW = ow;
+  a->IH = d->ih;
+  a->IW = d->iw;
+  a->K = d->k;
+  a->S = d->s;
+  a->D = d->d;
+  a->PT = (int32_t)d->pad[0];
+  a->PL = (int32_t)d->pad[1];
+  a->fd_ohw = aih::make_fastdiv(oh * ow);
+  a->fd_ow = aih::make_fastdiv(ow);
+  a->act = d->act;
+  a->has_res = d->residual ? 1 : 0;
+  conv_stream_tile(a, d->dt, shape);
+  return conv_stream_grid_ok(*a);
 }
 
 // ---------------------------------------------------------------- fused inverted-residual block
@@ -692,7 +845,7 @@ int plan_ir_head(const aih_ir_block_desc *d, const aih_pw_desc *h, uint32_t *oh,
   if (h->n != d->n || h->m != *oh * *ow || h->kg != d->cout / 4 || h->ng != 1 || h->residual)
     return fail("ir_block_head: the head must read the block's output (same n and pixels, kg = cout / 4) and "
                 "have at most 4 outputs (ng 1) and no residual");
-  if (pw_route(h) != PW_ROWS || aih::pw_narrow_group(h->kg) != 16)
+  if (pw_base_route(h) != PW_ROWS || aih::pw_narrow_group(h->kg) != 16)
     return fail("ir_block_head: the head must be on the narrow route with 16 lanes a pixel (AUTO, splitk 0, "
                 "kg >= 16)");
   if (d->kernel != AIH_IR_KERNEL_AUTO && d->kernel != AIH_IR_KERNEL_SPLIT)
@@ -718,7 +871,19 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out) {
     if (check_pw(d)) return AIH_ERR;
     if (!out) return fail("null plan");
     const uint64_t M = (uint64_t)d->n * d->m;
-    switch (pw_route(d)) {
+    const int base = pw_base_route(d);
+    aih::ConvStreamArgs ca;
+    aih::ConvStreamShape cs;
+    size_t need;
+    if (pw_dma_plan(d, base, &ca, &cs, &need)) {
+      // what a direct kernel would take (up to 64 outputs) is reported as its
+      // 32 pixels a wavefront, the rest as the workgroup's tile
+      const uint32_t grid = ca.mtiles * ca.ntiles;
+      *out = base == PW_TILED ? aih_plan{AIH_VAR_TILE, 1, aih::conv_stream_bm(cs), aih::conv_stream_bn(cs), grid, need}
+                              : aih_plan{AIH_VAR_DIRECT, 1, 32, ca.N4 <= 32 ? 32u : 64u, grid, 0};
+      return AIH_OK;
+    }
+    switch (base) {
       case PW_ROWS: {
         // pw_narrow_group(kg) lanes per pixel: 256 / that many pixels per workgroup
         const uint32_t ppb = 256 / aih::pw_narrow_group(d->kg);
@@ -774,7 +939,21 @@ int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *
     if ((d->residual != 0) != (res != nullptr)) return fail("pw: res must be given iff residual");
     if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 16) || !aligned(bias, 8) || (res && !aligned(res, 16)))
       return fail("pw: misaligned buffer (x, w, y, res need 16 bytes, bias 8)");
-    const int route = pw_route(d);
+    const int route = pw_base_route(d);
+    aih::ConvStreamArgs ca;
+    aih::ConvStreamShape cs;
+    size_t need;
+    if (pw_dma_plan(d, route, &ca, &cs, &need) && (need == 0 || (ws && ws_bytes >= need && aligned(ws, 16)))) {
+      // both operands streamed through LDS by DMA (a workspace too small for
+      // the plan is refused below, by the tiled GEMM)
+      ca.x = x;
+      ca.w = w;
+      ca.bias = bias;
+      ca.res = res;
+      ca.y = y;
+      const hipError_t e = aih::launch_conv_stream(ca, d->dt, cs, static_cast<hipStream_t>(stream));
+      return e == hipSuccess ? AIH_OK : fail(std::string("pw stream launch: ") + hipGetErrorString(e));
+    }
     if (route == PW_SPLITK) {
       // small M, long K: K split across the wavefronts of one workgroup,
       // reduced in LDS, one dispatch, no workspace
@@ -879,12 +1058,23 @@ int aih_conv_igemm_plan(const aih_igemm_desc *d, aih_plan *out) {
     }
     aih::IgDirectArgs da;
     if (ig_direct_plan(d, oh, ow, &da)) {
-      *out = aih_plan{AIH_VAR_DIRECT, 1, 32, da.N4 <= 32 ? 32u : 64u, aih::ig_direct_grid(da.nblk, da.nj, da.N4), 0};
+      // few pixels or whole 64-channel taps: the LDS-streamed kernel in the
+      // direct one's place, reported as the direct route
+      aih::ConvStreamArgs sa;
+      aih::ConvStreamShape sh;
+      uint32_t grid = aih::ig_direct_grid(da.nblk, da.nj, da.N4);
+      if (igemm_stream_plan(d, oh, ow, true, true, &sa, &sh)) grid = sa.mtiles * sa.ntiles;
+      *out = aih_plan{AIH_VAR_DIRECT, 1, 32, da.N4 <= 32 ? 32u : 64u, grid, 0};
       return AIH_OK;
     }
     GemmPlan g;
     if (plan_igemm(d, &g)) return AIH_ERR;
-    fill_plan(g, out);
+    aih::ConvStreamArgs sa;
+    aih::ConvStreamShape sh;
+    if (igemm_stream_plan(d, oh, ow, false, g.nsplit == 1, &sa, &sh))
+      *out = aih_plan{AIH_VAR_TILE, 1, aih::conv_stream_bm(sh), aih::conv_stream_bn(sh), sa.mtiles * sa.ntiles, g.ws};
+    else
+      fill_plan(g, out);
     return AIH_OK;
   });
 }
@@ -917,8 +1107,26 @@ int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const voi
       const hipError_t e = aih::launch_conv_stem(sa, d->dt, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("conv stem launch: ") + hipGetErrorString(e));
     }
+    // the workspace contract is the tiled GEMM's plan for what the direct
+    // kernel does not take: a call without it is refused there
     aih::IgDirectArgs da;
-    if (ig_direct_plan(d, oh, ow, &da)) {
+    const bool direct = ig_direct_plan(d, oh, ow, &da);
+    GemmPlan g{};
+    if (!direct && plan_igemm(d, &g)) return AIH_ERR;
+    const bool ws_ok = direct || g.ws == 0 || (ws && ws_bytes >= g.ws && aligned(ws, 16));
+    aih::ConvStreamArgs ca;
+    aih::ConvStreamShape sh;
+    if (ws_ok && igemm_stream_plan(d, oh, ow, direct, g.nsplit == 1, &ca, &sh)) {
+      // both operands streamed through LDS by DMA
+      ca.x = inputs[0];
+      ca.w = w;
+      ca.bias = bias;
+      ca.res = res;
+      ca.y = y;
+      const hipError_t e = aih::launch_conv_stream(ca, d->dt, sh, static_cast<hipStream_t>(stream));
+      return e == hipSuccess ? AIH_OK : fail(std::string("igemm stream launch: ") + hipGetErrorString(e));
+    }
+    if (direct) {
       // 3x3 with at most 64 output channels: weights resident in LDS,
       // activations straight into MFMA registers, no barriers after the load
       for (uint32_t i = 0; i < (d->nsrcs ? d->nsrcs : 1); ++i) da.src[i] = inputs[i];
@@ -930,8 +1138,6 @@ int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const voi
       const hipError_t e = aih::launch_ig_direct(da, d->dt, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("igemm direct launch: ") + hipGetErrorString(e));
     }
-    GemmPlan g;
-    if (plan_igemm(d, &g)) return AIH_ERR;
     aih::GemmArgs a;
     std::memset(&a, 0, sizeof(a));
     const uint32_t kg = div_ceil(d->cin, 4);
@@ -1211,8 +1417,7 @@ size_t aih_conv_workspace_size(const aih_conv_desc *d) {
   aih_dw_desc dw;
   GemmPlan g;
   const int r = conv_route(d, &pw, &ig, &dw);
-  if (r == 0 && !check_pw(&pw) && pw_route(&pw) != PW_TILED) return 0;
-  if (r == 0 && !check_pw(&pw) && !plan_pw(&pw, &g)) return g.ws;
+  if (r == 0 && !check_pw(&pw)) return pw_ws(&pw, pw_base_route(&pw));
   if (r == 1 && !check_igemm(&ig)) {
     uint32_t oh, ow;
     aih::IgDirectArgs da;

@@ -230,7 +230,14 @@ typedef struct {
  * (32 pixels per wavefront, operands from memory into registers); fp32 with
  * at least 256 input channels and enough pixels for eight 32 x 32 wavefront
  * units per CU runs a GEMM whose operands stream through LDS by DMA over
- * the whole K (reported as AIH_VAR_TILE with bm = 96, no workspace). */
+ * the whole K (reported as AIH_VAR_TILE with bm = 96, no workspace). With
+ * dt == wdt, whole 16-byte units (4 fp32 / 8 16-bit channels) a pixel, at
+ * least 4 of them, and more than 2048 pixels, a GEMM with both operands
+ * streamed through LDS runs at 16 bit what the tiled GEMM and most of what
+ * the direct kernel would (the latter still reported as AIH_VAR_DIRECT, 32
+ * pixels a wavefront), and at fp32 what the tiled GEMM would with K whole; the
+ * plan's workspace is still the tiled GEMM's, and a call without it is
+ * refused. */
 int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *bias,
                 const void *res, void *y, void *ws, size_t ws_bytes, aih_stream stream);
 int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);
@@ -240,7 +247,10 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);
  * over at most 3 input channels with cout 32 or 64, AIH_VAR_AUTO, splitk 0 and
  * dt == wdt -- the stem -- runs a dedicated kernel (all 27 tap-channel values
  * in one MFMA operand) instead of the planned implicit GEMM; it needs no
- * workspace. */
+ * workspace. Other one-input AIH_VAR_AUTO calls with dt == wdt and whole
+ * 16-byte units may run a GEMM with both operands streamed through LDS in the
+ * place of the tiled GEMM or of the direct 3x3 kernel; the plan reports the
+ * route and the workspace of the kernel it stands in for. */
 int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const void *w,
                    const void *bias, const void *res, void *y, void *ws, size_t ws_bytes,
                    aih_stream stream);
