@@ -21,6 +21,7 @@
 #include "conv_dw.h"
 #include "conv_gemm_launch.h"
 #include "conv_igemm_direct.h"
+#include "conv_ksplit.h"
 #include "conv_pw_direct.h"
 #include "conv_pw_narrow.h"
 #include "conv_pw_splitk.h"
@@ -703,6 +704,74 @@ bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool d
   return conv_stream_grid_ok(*a);
 }
 
+// A KxK call of few pixels on the kernel that splits K over a workgroup's
+// wavefronts (conv_ksplit.hip), or false: AIH_VAR_AUTO without a forced split,
+// the same storage for activations and weights, at most two input parts of
+// whole 16-byte units, buffers within 32-bit offsets, and few 16-pixel x
+// 16-channel blocks: at fp32 at most four a CU (72 -> 32 3x3 at 40x72, 360
+// blocks: 28.7 us on the direct kernel, 6.5 here; 64 -> 64, 720: 16.1 -> 7.7;
+// 256 -> 256 at 10x18 b4, 720: 33.4 -> 21.8; 128 -> 128 at 40x72, 1440: 29.5
+// there, 29.0 here, 64 -> 64 b4, 2880: 17.2 there, 24.5 here), at 16 bit two
+// (128 -> 128 at 20x36, 360: 12.2 -> 5.7, 72 -> 32, 360: 7.1 -> 4.8; 64 -> 64,
+// 720: 6.4 there, 6.3 here, 16 -> 48 b8, 1080: 6.3 there, 6.8 here).
+bool igemm_ksplit_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::ConvKsplitArgs *a) {
+  if (d->variant != AIH_VAR_AUTO || d->splitk != 0 || d->dt != d->wdt || d->k > aih::kConvKsplitMaxK) return false;
+  const uint32_t n4 = div_ceil(d->cout, 4) * 4, nparts = d->nsrcs ? d->nsrcs : 1;
+  if (nparts > 2) return false;
+  const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;
+  const uint64_t M = (uint64_t)d->n * oh * ow, nblk = div_ceil(n4, 16);
+  if ((M + 15) / 16 * nblk > aih::device_cus() * (d->dt == AIH_F32 ? 4ull : 2ull)) return false;
+  std::memset(a, 0, sizeof(*a));
+  uint32_t kg0 = 0;
+  for (uint32_t i = 0; i < nparts; ++i) {
+    const uint32_t kgi = div_ceil(d->nsrcs ? d->srcs[i].c : d->cin, 4);
+    const uint32_t stride = d->nsrcs ? d->srcs[i].stride_c / 4 : kgi;
+    const uint32_t off = d->nsrcs ? d->srcs[i].c_off / 4 : 0;
+    if (kgi % ku || stride % ku || off % ku) return false;
+    const uint64_t bytes = (uint64_t)d->n * d->ih * d->iw * stride * 4 * es;
+    if (bytes >= 0x80000000ull) return false;
+    a->src_bytes[i] = (uint32_t)bytes;
+    a->stride_u[i] = stride / ku;
+    a->off_u[i] = off / ku;
+    a->nu[i] = kgi / ku;
+    a->kg_first[i] = kg0;
+    kg0 += kgi;
+    a->st += div_ceil(a->nu[i], 4);
+    if (i == 0) a->st0 = a->st;
+  }
+  if (nparts == 1) {
+    a->src_bytes[1] = a->src_bytes[0];
+    a->stride_u[1] = a->stride_u[0];
+  }
+  a->KGP = div_ceil(div_ceil(d->cin, 4), 4) * 4;
+  const uint64_t wb = (uint64_t)d->k * d->k * a->KGP * n4 * 4 * es;
+  if (wb >= 0x80000000ull) return false;
+  a->w_bytes = (uint32_t)wb;
+  a->N4 = n4;
+  a->M = (uint32_t)M;
+  a->OHW = oh * ow;
+  a->OW = ow;
+  a->IH = d->ih;
+  a->IW = d->iw;
+  a->K = d->k;
+  a->S = d->s;
+  a->D = d->d;
+  a->PT = (int32_t)d->pad[0];
+  a->PL = (int32_t)d->pad[1];
+  a->items = d->k * d->k * a->st;
+  a->per = div_ceil(a->items, aih::kConvKsplitWaves);
+  a->nblk = (uint32_t)nblk;
+  a->act = d->act;
+  a->has_res = d->residual ? 1 : 0;
+  a->nxcd = aih::device_xcds();
+  a->fd_ohw = aih::make_fastdiv(oh * ow);
+  a->fd_ow = aih::make_fastdiv(ow);
+  a->fd_nblk = aih::make_fastdiv(a->nblk);
+  a->fd_st = aih::make_fastdiv(a->st);
+  a->fd_k = aih::make_fastdiv(d->k);
+  return true;
+}
+
 // ---------------------------------------------------------------- fused inverted-residual block
 
 int check_ir(const aih_ir_block_desc *d, uint32_t *oh, uint32_t *ow) {
@@ -1114,6 +1183,18 @@ int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const voi
     GemmPlan g{};
     if (!direct && plan_igemm(d, &g)) return AIH_ERR;
     const bool ws_ok = direct || g.ws == 0 || (ws && ws_bytes >= g.ws && aligned(ws, 16));
+    aih::ConvKsplitArgs ka;
+    if (ws_ok && igemm_ksplit_plan(d, oh, ow, &ka)) {
+      // few pixels: K over a workgroup's wavefronts
+      for (uint32_t i = 0; i < nin; ++i) ka.src[i] = inputs[i];
+      if (nin == 1) ka.src[1] = ka.src[0];
+      ka.w = w;
+      ka.bias = bias;
+      ka.res = res;
+      ka.y = y;
+      const hipError_t e = aih::launch_conv_ksplit(ka, d->dt, static_cast<hipStream_t>(stream));
+      return e == hipSuccess ? AIH_OK : fail(std::string("igemm ksplit launch: ") + hipGetErrorString(e));
+    }
     aih::ConvStreamArgs ca;
     aih::ConvStreamShape sh;
     if (ws_ok && igemm_stream_plan(d, oh, ow, direct, g.nsplit == 1, &ca, &sh)) {

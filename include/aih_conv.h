@@ -249,8 +249,9 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);
  * in one MFMA operand) instead of the planned implicit GEMM; it needs no
  * workspace. Other one-input AIH_VAR_AUTO calls with dt == wdt and whole
  * 16-byte units may run a GEMM with both operands streamed through LDS in the
- * place of the tiled GEMM or of the direct 3x3 kernel; the plan reports the
- * route and the workspace of the kernel it stands in for. */
+ * place of the tiled GEMM or of the direct 3x3 kernel, and ones of at most two
+ * inputs and few pixels a kernel whose workgroups split K on chip; the plan
+ * reports the route and the workspace of the kernel they stand in for. */
 int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const void *w,
                    const void *bias, const void *res, void *y, void *ws, size_t ws_bytes,
                    aih_stream stream);
