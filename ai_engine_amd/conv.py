@@ -20,6 +20,7 @@ import ctypes as C
 import enum
 import os
 from dataclasses import dataclass, field
+from operator import attrgetter
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libaih_conv.so")
@@ -244,7 +245,8 @@ def _stream(stream) -> int | None:
     if stream is None:
         import torch
 
-        return torch.cuda.current_stream().cuda_stream
+        # torch.cuda.current_stream().cuda_stream without its Stream object
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -256,6 +258,27 @@ def _workspace(nbytes: int, ws, device):
     import torch
 
     return torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=device)
+
+
+def _desc_of(spec, fields):
+    """spec.desc(), built again only when a field's value differs from the last
+    run's (a launch's descriptor takes as long to build as the rest of the
+    call). The values are compared, so a changed spec is never run with an old
+    descriptor; a spec with a field that can change in place (a list), or of a
+    class derived from these, builds it every time. The C side only reads it."""
+    key = fields(spec)
+    last = spec.__dict__.get("_last_desc")
+    if last is not None and last[0] == key:
+        return last[1]
+    d = spec.desc()
+    if type(spec) in (ConvOp, IrBlockSpec, DwPwSpec) and all(
+            type(v) in _PLAIN or isinstance(v, enum.IntEnum) or
+            (type(v) is tuple and all(type(e) is int for e in v)) for v in key):
+        spec.__dict__["_last_desc"] = (key, d)
+    return d
+
+
+_PLAIN = {int, bool, type(None)}
 
 
 def _device_of(t):
@@ -449,11 +472,15 @@ class ConvOp:
         return p
 
     def run(self, x, w, bias, res, y, ws=None, stream=None):
-        nb = self.workspace_bytes()
+        L, d = lib(), C.byref(_desc_of(self, _CONV_FIELDS))
+        nb = L.aih_conv_workspace_size(d)
         ws = _workspace(nb, ws, _device_of(y))
-        _check(lib().aih_conv(C.byref(self.desc()), _ptr(x), _ptr(w), _ptr(bias), _ptr(res), _ptr(y), _ptr(ws),
-                              nb if ws is not None else 0, _stream(stream)))
+        _check(L.aih_conv(d, _ptr(x), _ptr(w), _ptr(bias), _ptr(res), _ptr(y), _ptr(ws),
+                          nb if ws is not None else 0, _stream(stream)))
         return y
+
+
+_CONV_FIELDS = attrgetter(*ConvOp.__dataclass_fields__)
 
 
 @dataclass
@@ -502,10 +529,13 @@ class IrBlockSpec:
         return lib().aih_ir_block_plan(C.byref(self.desc()), C.byref(p)) == 0
 
     def run(self, x, w_expand, b_expand, w_dw, b_dw, w_project, b_project, res, y, stream=None):
-        _check(lib().aih_ir_block(C.byref(self.desc()), _ptr(x), _ptr(w_expand), _ptr(b_expand), _ptr(w_dw),
-                                  _ptr(b_dw), _ptr(w_project), _ptr(b_project), _ptr(res), _ptr(y),
+        _check(lib().aih_ir_block(C.byref(_desc_of(self, _IR_FIELDS)), _ptr(x), _ptr(w_expand), _ptr(b_expand),
+                                  _ptr(w_dw), _ptr(b_dw), _ptr(w_project), _ptr(b_project), _ptr(res), _ptr(y),
                                   _stream(stream)))
         return y
+
+
+_IR_FIELDS = attrgetter(*IrBlockSpec.__dataclass_fields__)
 
 
 @dataclass
@@ -612,9 +642,12 @@ class DwPwSpec:
         return lib().aih_conv_dwpw_plan(C.byref(self.desc()), C.byref(p)) == 0
 
     def run(self, x, w_dw, b_dw, w_pw, b_pw, res, y, stream=None):
-        _check(lib().aih_conv_dwpw(C.byref(self.desc()), _ptr(x), _ptr(w_dw), _ptr(b_dw), _ptr(w_pw), _ptr(b_pw),
-                                   _ptr(res), _ptr(y), _stream(stream)))
+        _check(lib().aih_conv_dwpw(C.byref(_desc_of(self, _DWPW_FIELDS)), _ptr(x), _ptr(w_dw), _ptr(b_dw), _ptr(w_pw),
+                                   _ptr(b_pw), _ptr(res), _ptr(y), _stream(stream)))
         return y
+
+
+_DWPW_FIELDS = attrgetter(*DwPwSpec.__dataclass_fields__)
 
 
 def pack_nhwc_device(x, n, h, w, c, dt: DType, y, stream=None):
