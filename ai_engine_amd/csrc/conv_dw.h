@@ -18,5 +18,8 @@ struct DwArgs {
 
 hipError_t launch_conv_dw(const DwArgs &a, int dt, hipStream_t st);
 hipError_t launch_pack_nhwc(const float *x, uint64_t px, uint32_t c, int dt, void *y, hipStream_t st);
+// px pixels of c channels: x points at the first one's first channel
+hipError_t launch_unpack_nhwc(const void *x, uint32_t px, uint32_t c, uint32_t stride_c, int dt, float *y,
+                              hipStream_t st);
 
 }  // namespace aih

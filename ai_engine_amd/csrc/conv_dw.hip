@@ -1,4 +1,4 @@
-// conv_dw.hip -- depthwise KxK conv and the device-side NHWC -> NHWC-C4 pack.
+// conv_dw.hip -- depthwise KxK conv and the device-side NHWC <-> NHWC-C4 pack.
 //
 // Depthwise is HBM-bound (2 flops per weight per pixel, no reuse across
 // channels). The arithmetic follows the reference depthwise path
@@ -348,6 +348,43 @@ hipError_t launch_pack_nhwc(const float *x, uint64_t px, uint32_t c, int dt, voi
     case DT_BF16: hipLaunchKernelGGL(pack_nhwc_kernel<DT_BF16>, grid, dim3(256), 0, st, x, px, c, y); break;
     default: return hipErrorInvalidValue;
   }
+  return hipGetLastError();
+}
+
+// Pixels of stride_c storage channels, from channel c_off on -> logical fp32
+// NHWC; one value per thread. The way back of a result to the host: with
+// the padding gone before the copy (and 16-bit values widened, exactly) the
+// copy is the caller's bytes and the host has no pass over them (160x288x2
+// fp32 b1: 368 KB instead of 737, and no second buffer).
+template <int DT>
+__global__ __launch_bounds__(256) void unpack_nhwc_kernel(const typename Storage<DT>::T *__restrict__ x,
+                                                          uint32_t stride_c, FastDiv fd_c, uint32_t total,
+                                                          float *__restrict__ y) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t p = fdiv(i, fd_c);
+  const typename Storage<DT>::T v = x[(size_t)p * stride_c + (i - p * fd_c.d)];
+  if constexpr (DT == DT_F32) y[i] = v;
+  else if constexpr (DT == DT_F16) y[i] = f16_to_f32(v);
+  else y[i] = bf16_to_f32(v);
+}
+
+hipError_t launch_unpack_nhwc(const void *x, uint32_t px, uint32_t c, uint32_t stride_c, int dt, float *y,
+                              hipStream_t st) {
+  const uint64_t n = (uint64_t)px * c;
+  if (n == 0 || n > 0x7fffff00u) return hipErrorInvalidValue;
+  const FastDiv fd = make_fastdiv(c);
+  const dim3 grid((unsigned)((n + 255) / 256));
+#define AIH_UNPACK(DT)                                                                                      \
+  hipLaunchKernelGGL(unpack_nhwc_kernel<DT>, grid, dim3(256), 0, st, static_cast<const Storage<DT>::T *>(x), \
+                     stride_c, fd, (uint32_t)n, y)
+  switch (dt) {
+    case DT_F32: AIH_UNPACK(DT_F32); break;
+    case DT_F16: AIH_UNPACK(DT_F16); break;
+    case DT_BF16: AIH_UNPACK(DT_BF16); break;
+    default: return hipErrorInvalidValue;
+  }
+#undef AIH_UNPACK
   return hipGetLastError();
 }
 

@@ -26,12 +26,14 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
 #include "../../include/aih_model.h"
 #include "aih_device.h"
 #include "capi_util.h"
+#include "conv_dw.h"
 #include "sw_format.h"
 
 namespace aih {
@@ -72,38 +74,6 @@ uint16_t f32_to_bf16_bits(float f) {
   return (uint16_t)(x >> 16);
 }
 
-float f16_bits_to_f32(uint16_t h) {
-  const uint32_t sign = (uint32_t)(h & 0x8000u) << 16;
-  uint32_t e = (h >> 10) & 0x1fu, m = h & 0x3ffu;
-  uint32_t x;
-  if (e == 0) {
-    if (m == 0) {
-      x = sign;
-    } else {  // subnormal: normalise
-      e = 113;
-      while (!(m & 0x400u)) {
-        m <<= 1;
-        --e;
-      }
-      x = sign | (e << 23) | ((m & 0x3ffu) << 13);
-    }
-  } else if (e == 31) {
-    x = sign | 0x7f800000u | (m << 13);
-  } else {
-    x = sign | ((e + 112) << 23) | (m << 13);
-  }
-  float f;
-  std::memcpy(&f, &x, 4);
-  return f;
-}
-
-float bf16_bits_to_f32(uint16_t h) {
-  const uint32_t x = (uint32_t)h << 16;
-  float f;
-  std::memcpy(&f, &x, 4);
-  return f;
-}
-
 int hip_fail(const char *what, hipError_t e) { return api_fail(std::string(what) + ": " + hipGetErrorString(e)); }
 
 // A JSON string literal of s (quotes, backslashes and control characters escaped).
@@ -129,6 +99,8 @@ std::string json_quote(const std::string &s) {
 
 using namespace aih;
 
+constexpr size_t kReadFloats = 16u << 20;
+
 struct aih_model {
   sw::Model g;
   uint32_t n = 1;
@@ -148,6 +120,11 @@ struct aih_model {
   size_t ws_bytes = 0;
   float *staging = nullptr;
   size_t staging_floats = 0;
+  // read_output's logical fp32 values on their way to the host, an output (or
+  // kReadFloats of a larger tensor) at a time; one reader at a time holds it
+  float *reading = nullptr;
+  size_t read_floats = 0;
+  std::mutex read_mutex;
   std::vector<std::function<int(hipStream_t)>> launches;  // per op; empty for a fused block's later ops
   size_t device_bytes = 0;
   uint32_t flags = 0;
@@ -1363,6 +1340,12 @@ aih_model *aih_model_load_ex(const void *bytes, size_t len, uint32_t n, int32_t 
     for (uint32_t t : m->g.inputs)
       m->staging_floats = std::max(m->staging_floats, (size_t)n * m->g.tensors[t].h * m->g.tensors[t].w * m->g.tensors[t].c);
     if (m->staging_floats) m->staging = static_cast<float *>(m->dalloc(m->staging_floats * 4));
+    // 64 MB at most, and a pixel of any tensor
+    for (uint32_t t : m->g.outputs)
+      m->read_floats = std::max(m->read_floats, (size_t)n * m->g.tensors[t].h * m->g.tensors[t].w * m->g.tensors[t].c);
+    m->read_floats = std::min(std::max<size_t>(m->read_floats, 1u << 16), kReadFloats);
+    for (const auto &t : m->g.tensors) m->read_floats = std::max<size_t>(m->read_floats, t.c);
+    m->reading = static_cast<float *>(m->dalloc(m->read_floats * 4));
     lower(m.get());
     if (m->ws_bytes) m->ws = m->dalloc(m->ws_bytes);
     fuse_stem_launch(m.get());
@@ -1457,27 +1440,29 @@ int aih_model_read_output(aih_model *m, const char *name, float *host_nhwc, size
     const size_t want = (size_t)m->n * t.h * t.w * t.c;
     if (count != want) return api_fail("read_output: expected " + std::to_string(want) + " floats");
     const aih_model::View &v = m->views[tid];
-    hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    // a stream under capture cannot be waited for: the wait says so, before
+    // anything is recorded
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(s, &cap);
+    if (e == hipSuccess && cap != hipStreamCaptureStatusNone) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail("read_output", e);
-    std::vector<uint8_t> buf(v.bytes);
-    e = hipMemcpy(buf.data(), v.base, v.bytes, hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return hip_fail("read_output copy", e);
-    const size_t es = es_of(m->dt);
-    const size_t px = (size_t)m->n * t.h * t.w;
-    for (size_t p = 0; p < px; ++p)
-      for (uint32_t ch = 0; ch < t.c; ++ch) {
-        const uint8_t *q = buf.data() + (p * v.stride_c + v.c_off + ch) * es;
-        float f;
-        if (m->dt == AIH_F32) {
-          std::memcpy(&f, q, 4);
-        } else {
-          uint16_t h;
-          std::memcpy(&h, q, 2);
-          f = m->dt == AIH_F16 ? f16_bits_to_f32(h) : bf16_bits_to_f32(h);
-        }
-        host_nhwc[p * t.c + ch] = f;
-      }
-    return AIH_OK;
+    // unpacked on the device behind the work that writes the tensor, then
+    // copied straight to the caller (one frame of the real segmentation model,
+    // 160x288x2 fp32, host memory in and out: 331 us a call with the padded
+    // copy and the host's pass over it, 300 here)
+    std::lock_guard<std::mutex> lock(m->read_mutex);
+    const size_t px = (size_t)m->n * t.h * t.w, step = m->read_floats / t.c;
+    for (size_t p = 0; p < px && e == hipSuccess; p += step) {
+      const size_t k = std::min(step, px - p);
+      const char *src = v.base + (p * v.stride_c + v.c_off) * es_of(m->dt);
+      e = launch_unpack_nhwc(src, (uint32_t)k, t.c, v.stride_c, m->dt, m->reading, s);
+      if (e == hipSuccess)
+        e = hipMemcpyAsync(host_nhwc + p * t.c, m->reading, k * t.c * 4, hipMemcpyDeviceToHost, s);
+    }
+    const hipError_t w = hipStreamSynchronize(s);  // nothing writes to the caller after the return
+    if (e == hipSuccess) e = w;
+    return e == hipSuccess ? AIH_OK : hip_fail("read_output", e);
   });
 }
 
