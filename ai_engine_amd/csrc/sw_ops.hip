@@ -3,11 +3,10 @@
 // reads it), global average pool, binary elementwise with the six SwOperand
 // kinds, channel concat. All are streaming kernels over NHWC-C4 with fp32
 // arithmetic on the storage dtype: one thread per output vec4 (gpool: a
-// workgroup per image and channel group; resize: a workgroup per pair of
-// output rows, its threads over the rows' vec4s); the grids cover the output
-// exactly and every index is checked against it. Output vec4 counts are kept
-// below 2^32 (checked on the host) so the index decomposition is 32-bit with
-// precomputed divisors.
+// workgroup per image and channel group; resize: one thread per vec4 of a pair
+// of output rows); the grids cover the output exactly and every index is
+// checked against it. Output vec4 counts are kept below 2^32 (checked on the
+// host) so the index decomposition is 32-bit with precomputed divisors.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -89,9 +88,8 @@ __device__ __forceinline__ f32x4 part_load(const void *base, size_t idx) {
 // One workgroup per group of one or two consecutive output rows of an image
 // (`off` = 1: row 0 alone, then rows 2k - 1, 2k -- the pairs a 2x half-pixel
 // upsample maps to one source row pair; `off` = 0: rows 2k, 2k + 1). The
-// group's source rows and y weights are computed once, and the threads stride
-// over the row's ow * cg output vec4s (stores of consecutive threads are
-// consecutive). Part p with bit p of parts.resized set is read at ih x iw and
+// group's source rows and y weights are uniform, and consecutive threads take
+// consecutive ones of the row's ow * cg output vec4s. Part p with bit p of parts.resized set is read at ih x iw and
 // blended from its four taps -- when both rows of the group have the same
 // two source rows, their x blends (top, bot) are computed once and only the y
 // blend differs: the same operations on the same values as two separate rows
@@ -129,15 +127,20 @@ __device__ __forceinline__ void resize_vec(const PartArg &pa, bool resized, uint
     if (k0 + l >= pa.c) va[l] = vb[l] = 0.0f;
 }
 
-// Rows of up to 1024 vec4s take one thread per vec4 (the block rounded up
-// to whole wavefronts); longer rows 256 threads that stride over the row.
+// One thread per vec4 of the row pair: rows of up to 1024 vec4s in one
+// workgroup (rounded up to whole wavefronts), longer ones in `bpr` workgroups of
+// about 512. (A thread's loads wait for its index arithmetic and the part's
+// branch, so threads that stride over a long row wait once per turn: with 256
+// of them 80x144x44 from 40x72x32 + 12 took 12.4 us fp32 b1, here 4.0.)
 template <int DT, bool O32>
 __global__ __launch_bounds__(1024) void resize_kernel(Parts parts, uint32_t ih, uint32_t iw, uint32_t oh,
                                                       uint32_t ow, float sy, float sx, int mode, uint32_t cg_out,
                                                       FastDiv fd_cg, uint32_t groups, FastDiv fd_groups,
-                                                      uint32_t off, void *y) {
-  const uint32_t img = fdiv(blockIdx.x, fd_groups);
-  const uint32_t k = blockIdx.x - img * groups;
+                                                      uint32_t off, FastDiv fd_bpr, void *y) {
+  const uint32_t grp = fdiv(blockIdx.x, fd_bpr);
+  const uint32_t j0 = (blockIdx.x - grp * fd_bpr.d) * blockDim.x;
+  const uint32_t img = fdiv(grp, fd_groups);
+  const uint32_t k = grp - img * groups;
   const uint32_t ra = off ? (k == 0 ? 0u : 2 * k - 1) : 2 * k;
   const bool two = !(off && k == 0) && ra + 1 < oh;
   const Coord ca = resize_coord(ra, sy, mode, ih);
@@ -147,20 +150,20 @@ __global__ __launch_bounds__(1024) void resize_kernel(Parts parts, uint32_t ih, 
   const size_t a0 = (ib + ca.i0) * iw, a1 = (ib + ca.i1) * iw, b0 = (ib + cb.i0) * iw, b1 = (ib + cb.i1) * iw;
   const size_t row_a = (size_t)img * oh + ra;  // output (and plain part) rows
   const uint32_t nrow = ow * cg_out;
-  for (uint32_t j = threadIdx.x; j < nrow; j += blockDim.x) {
-    const uint32_t ox = fdiv(j, fd_cg);
-    const uint32_t g4 = (j - ox * cg_out) * 4;
-    f32x4 va = {}, vb = {};
-    for (uint32_t p = 0; p < parts.n; ++p) {
-      const PartArg &pa = parts.v[p];
-      const uint32_t end = p + 1 < parts.n ? parts.v[p + 1].out_c0 : 0xffffffffu;
-      if (g4 >= pa.out_c0 && g4 < end)
-        resize_vec<DT, O32>(pa, (parts.resized >> p) & 1u, g4 - pa.out_c0, ox, row_a * ow, (row_a + 1) * ow, two,
-                            shared, a0, a1, b0, b1, ca, cb, sx, mode, iw, va, vb);
-    }
-    Vec4IO<DT>::store(y, row_a * nrow + j, va);
-    if (two) Vec4IO<DT>::store(y, (row_a + 1) * nrow + j, vb);
+  const uint32_t j = j0 + threadIdx.x;
+  if (j >= nrow) return;
+  const uint32_t ox = fdiv(j, fd_cg);
+  const uint32_t g4 = (j - ox * cg_out) * 4;
+  f32x4 va = {}, vb = {};
+  for (uint32_t p = 0; p < parts.n; ++p) {
+    const PartArg &pa = parts.v[p];
+    const uint32_t end = p + 1 < parts.n ? parts.v[p + 1].out_c0 : 0xffffffffu;
+    if (g4 >= pa.out_c0 && g4 < end)
+      resize_vec<DT, O32>(pa, (parts.resized >> p) & 1u, g4 - pa.out_c0, ox, row_a * ow, (row_a + 1) * ow, two,
+                          shared, a0, a1, b0, b1, ca, cb, sx, mode, iw, va, vb);
   }
+  Vec4IO<DT>::store(y, row_a * nrow + j, va);
+  if (two) Vec4IO<DT>::store(y, (row_a + 1) * nrow + j, vb);
 }
 
 // ---------------------------------------------------------------- gpool
@@ -339,7 +342,8 @@ int launch_resize(const char *what, uint32_t n, uint32_t ih, uint32_t iw, uint32
   const uint64_t total = rows * ow * cg;
   if (total > 0xffffff00ull || rows > 0x7fffffffull) return api_fail(w + ": output too large");
   const uint32_t nrow = ow * cg;
-  const uint32_t threads = nrow <= 1024 ? (nrow + 63) / 64 * 64 : 256u;
+  const uint32_t bpr = nrow <= 1024 ? 1u : (nrow + 511) / 512;
+  const uint32_t threads = ((nrow + bpr - 1) / bpr + 63) / 64 * 64;
   // every part's vec4s (its ih x iw or oh x ow pixels times stride_c / 4) below 4 GiB
   bool o32 = true;
   for (uint32_t i = 0; i < nsrcs; ++i) {
@@ -361,11 +365,12 @@ int launch_resize(const char *what, uint32_t n, uint32_t ih, uint32_t iw, uint32
   const uint32_t off = share[1] > share[0] ? 1u : 0u;
   const uint32_t groups = off ? 1 + oh / 2 : (oh + 1) / 2;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)(n * groups)), block(threads);
-  const FastDiv fcg = make_fastdiv(cg), fgr = make_fastdiv(groups);
+  if ((uint64_t)n * groups * bpr > 0x7fffffffull) return api_fail(w + ": output too large");
+  const dim3 grid((unsigned)(n * groups * bpr)), block(threads);
+  const FastDiv fcg = make_fastdiv(cg), fgr = make_fastdiv(groups), fbpr = make_fastdiv(bpr);
 #define AIH_RESIZE_LAUNCH(D, O)                                                                                  \
   hipLaunchKernelGGL((resize_kernel<D, O>), grid, block, 0, st, parts, ih, iw, oh, ow, sy, sx, (int)mode, cg, fcg, \
-                     groups, fgr, off, y)
+                     groups, fgr, off, fbpr, y)
   switch (dt) {
     case AIH_F32: if (o32) AIH_RESIZE_LAUNCH(DT_F32, true); else AIH_RESIZE_LAUNCH(DT_F32, false); break;
     case AIH_F16: if (o32) AIH_RESIZE_LAUNCH(DT_F16, true); else AIH_RESIZE_LAUNCH(DT_F16, false); break;
