@@ -440,6 +440,21 @@ size_t pw_ws(const aih_pw_desc *d, int base) {
   return base == PW_TILED && !plan_pw(d, &g) ? g.ws : 0;
 }
 
+// A call of the tiled GEMM's (fewer than 64 input channels, more outputs than
+// the direct kernel holds) that the one-dispatch split-K kernel runs: at most
+// kPwSplitkMaxM pixels and 24 of its 16-pixel x 16-channel blocks a CU (fp32 48
+// -> 192 at 10x18, 144 blocks: 6.4 us tiled, 2.7 here; 32 -> 960 at 1440
+// pixels, 5400: 7.0, 5.4; f16 48 -> 192 4.9, 2.6; 32 -> 960 at 1984 pixels,
+// 7440: 5.1, 5.0). The workspace is still the tiled GEMM's plan: a call without
+// it goes there and is refused.
+bool pw_short_k(const aih_pw_desc *d, const void *ws, size_t ws_bytes) {
+  if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || !pw_splitk_shape(d)) return false;
+  const uint64_t M = (uint64_t)d->n * d->m;
+  if ((M + 15) / 16 * (d->ng / 4) > 24ull * aih::device_cus()) return false;
+  GemmPlan g;
+  return !plan_pw(d, &g) && (g.ws == 0 || (ws && ws_bytes >= g.ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0));
+}
+
 // Arguments of the one-dispatch split-K kernel and its K chunks (waves).
 aih::PwSplitkArgs pw_splitk_args(const aih_pw_desc *d, uint32_t *waves) {
   aih::PwSplitkArgs a;
@@ -1023,9 +1038,9 @@ int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *
       const hipError_t e = aih::launch_conv_stream(ca, d->dt, cs, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("pw stream launch: ") + hipGetErrorString(e));
     }
-    if (route == PW_SPLITK) {
-      // small M, long K: K split across the wavefronts of one workgroup,
-      // reduced in LDS, one dispatch, no workspace
+    if (route == PW_SPLITK || (route == PW_TILED && pw_short_k(d, ws, ws_bytes))) {
+      // small M: K split across the wavefronts of one workgroup, reduced in
+      // LDS, one dispatch, no workspace
       uint32_t waves;
       aih::PwSplitkArgs a = pw_splitk_args(d, &waves);
       a.x = x;

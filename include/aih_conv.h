@@ -235,9 +235,10 @@ typedef struct {
  * least 4 of them, and more than 2048 pixels, a GEMM with both operands
  * streamed through LDS runs at 16 bit what the tiled GEMM and most of what
  * the direct kernel would (the latter still reported as AIH_VAR_DIRECT, 32
- * pixels a wavefront), and at fp32 what the tiled GEMM would with K whole; the
- * plan's workspace is still the tiled GEMM's, and a call without it is
- * refused. */
+ * pixels a wavefront), and at fp32 what the tiled GEMM would with K whole; and
+ * up to 2048 pixels the split-K kernel runs the tiled GEMM's calls of few
+ * 16 x 16 output blocks. The plan is still the tiled GEMM's for both, its
+ * workspace too, and a call without it is refused. */
 int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *bias,
                 const void *res, void *y, void *ws, size_t ws_bytes, aih_stream stream);
 int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);

@@ -1,5 +1,5 @@
 """The KxK conv whose workgroups split K over their wavefronts
-(csrc/conv_ksplit.hip) against the oracle, at the edges of its blocks: ragged
+(csrc/conv_ksplit.hip), and short pointwise calls on the pointwise one, against the oracle, at the edges of its blocks: ragged
 pixel and channel blocks, taps outside the image, units past a part, (tap,
 step) pairs that do not divide by the wavefronts, two input parts, and both
 sides of its block limit. Tolerances are those of the kernels it stands beside:
@@ -46,6 +46,21 @@ def test_igemm(case, dt):
     r = G.run_igemm(ih, iw, cin, cout, k, s, pad, act, res, dt, 9700 + cin, n=n, d=d)
     assert not np.isnan(np.asarray(r.got)).any(), case
     check(f"igemm {case}", G.rel_err(r.got, r.want_r), dt)
+
+
+# h, w, cin, cout, n: pointwise calls of the tiled GEMM's that the one-dispatch
+# split-K kernel runs
+PW = [(1, 1, 4, 80, 1), (10, 18, 48, 192, 1), (7, 5, 44, 144, 3), (23, 31, 60, 112, 2), (32, 64, 8, 768, 1),
+      (32, 64, 12, 784, 1)]  # both sides of 24 blocks a CU of 256
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", PW, ids=lambda c: "x".join(map(str, c)))
+def test_pointwise_short_k(case, dt):
+    h, w, cin, cout, n = case
+    r = G.run_pw(h, w, cin, cout, "relu6", True, dt, 9850 + cin, n=n)
+    assert not np.isnan(np.asarray(r.got)).any(), case
+    check(f"pw {case} {r.plan}", G.rel_err(r.got, r.want_r), dt)
 
 
 @pytest.mark.parametrize("dt", [F32, F16], ids=["f32", "f16"])
