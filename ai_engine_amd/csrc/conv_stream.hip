@@ -376,10 +376,13 @@ hipError_t launch_inst(const ConvStreamArgs &a, hipStream_t st) {
 
 template <int DT>
 hipError_t launch_dt(const ConvStreamArgs &a, const ConvStreamShape &s, hipStream_t st) {
+  // pointwise: output pixel m reads input pixel m (a 1x1 conv with a stride or
+  // padding is an implicit GEMM of one tap)
+  const bool pw = a.K == 1 && a.S == 1 && a.PT == 0 && a.PL == 0 && a.OW == a.IW && a.OHW == a.IH * a.IW;
 #define AIH_CS_CASE(WM, WN, TM, TN, BKU, NST)                                                         \
   if (s.wm == WM && s.wn == WN && s.tm == TM && s.tn == TN && s.bku == BKU && s.nst == NST)            \
-    return a.K == 1 ? launch_inst<DT, WM, WN, TM, TN, BKU, NST, false>(a, st)                         \
-                    : launch_inst<DT, WM, WN, TM, TN, BKU, NST, true>(a, st);
+    return pw ? launch_inst<DT, WM, WN, TM, TN, BKU, NST, false>(a, st)                               \
+              : launch_inst<DT, WM, WN, TM, TN, BKU, NST, true>(a, st);
   AIH_CS_CASE(2, 2, 2, 2, 4, 2)
   AIH_CS_CASE(4, 1, 1, 3, 4, 3)
   AIH_CS_CASE(4, 1, 1, 2, 4, 3)

@@ -73,6 +73,24 @@ def test_igemm(case, dt):
     check(f"igemm {case}", G.run_igemm(ih, iw, cin, cout, k, s, pad, act, res, dt, 9300 + cin, n=n, d=d), dt)
 
 
+# ih, iw, cin, cout, s, d, pad, n: 1x1 convs through the KxK entry, past the
+# split-K kernel's block limit; only the last reads input pixel m for output m
+ONE_TAP = [(97, 101, 64, 68, 2, 1, (0, 0, 0, 0), 5),
+           (66, 61, 48, 100, 1, 1, (0, 1, 1, 0), 4),
+           (65, 63, 48, 100, 1, 1, (0, 0, 2, 0), 4),  # rows below the image only
+           (65, 63, 48, 100, 1, 2, (0, 0, 0, 1), 4),  # columns right of it only
+           (64, 64, 40, 72, 1, 1, (1, 0, 0, 1), 4),   # as many outputs as inputs, shifted
+           (199, 187, 328, 96, 3, 1, (2, 1, 0, 2), 3),  # stages of 8 units, pixels with no input
+           (65, 63, 72, 100, 1, 1, (0, 0, 0, 0), 4)]
+
+
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", ONE_TAP, ids=lambda c: "x".join(map(str, c[:6])))
+def test_one_tap_with_stride_and_padding(case, dt):
+    ih, iw, cin, cout, s, d, pad, n = case
+    check(f"1x1 {case}", G.run_igemm(ih, iw, cin, cout, 1, s, pad, "none", False, dt, 9350 + cin, n=n, d=d), dt)
+
+
 @pytest.mark.parametrize("dt", [F32, F16], ids=["f32", "f16"])
 def test_igemm_channel_view(dt):
     """Channels 8..71 of an 88-channel input: the pixel stride and offset of a
