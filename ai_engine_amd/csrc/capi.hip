@@ -728,9 +728,12 @@ bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool d
 // 256 -> 256 at 10x18 b4, 720: 33.4 -> 21.8; 128 -> 128 at 40x72, 1440: 29.5
 // there, 29.0 here, 64 -> 64 b4, 2880: 17.2 there, 24.5 here), at 16 bit two
 // (128 -> 128 at 20x36, 360: 12.2 -> 5.7, 72 -> 32, 360: 7.1 -> 4.8; 64 -> 64,
-// 720: 6.4 there, 6.3 here, 16 -> 48 b8, 1080: 6.3 there, 6.8 here).
+// 720: 6.4 there, 6.3 here, 16 -> 48 b8, 1080: 6.3 there, 6.8 here). Not under
+// AIH_IGEMM_NO_SPLIT, which keeps K whole.
 bool igemm_ksplit_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::ConvKsplitArgs *a) {
-  if (d->variant != AIH_VAR_AUTO || d->splitk != 0 || d->dt != d->wdt || d->k > aih::kConvKsplitMaxK) return false;
+  if (d->variant != AIH_VAR_AUTO || d->splitk != 0 || env_igemm_no_split() || d->dt != d->wdt ||
+      d->k > aih::kConvKsplitMaxK)
+    return false;
   const uint32_t n4 = div_ceil(d->cout, 4) * 4, nparts = d->nsrcs ? d->nsrcs : 1;
   if (nparts > 2) return false;
   const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;

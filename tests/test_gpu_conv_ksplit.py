@@ -5,6 +5,10 @@ step) pairs that do not divide by the wavefronts, two input parts, and both
 sides of its block limit. Tolerances are those of the kernels it stands beside:
 fp32 sums of at most 25 x 256 products (relative 1e-4), 16-bit storage with
 fp32 sums (two roundings of the result against the stored inputs)."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -99,3 +103,30 @@ def test_infinities_stay_in_their_taps():
     assert torch.isposinf(got[:2, :2]).all()
     got[:2, :2] = 0
     assert torch.isfinite(got).all()
+
+
+NO_SPLIT_PROBE = """
+import sys
+sys.path.insert(0, %r)
+import numpy as np
+from tests import gpu_util as G
+for dt in (0, 1, 2):
+    for cin, cout in ((128, 128), (64, 64)):
+        xs = [G.run_igemm(9, 16, cin, cout, 3, 1, [1] * 4, "relu", True, dt, 9950, splitk=k, refs=False).got for k in (0, 1)]
+        print(int(np.array_equal(*map(np.asarray, xs))), end=" ")
+"""
+
+
+def test_no_split_override_keeps_k_whole():
+    """Under AIH_IGEMM_NO_SPLIT=1 (read once per process) a call of few pixels
+    sums K whole: the bits of the forced split of 1. Without it the sums are
+    those of nine wavefronts, and the bits differ."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = []
+    for v in ("1", ""):
+        r = subprocess.run([sys.executable, "-c", NO_SPLIT_PROBE % root], capture_output=True, text=True, timeout=100,
+                           env=dict(os.environ, AIH_IGEMM_NO_SPLIT=v))
+        assert r.returncode == 0, r.stderr
+        got.append(r.stdout.split())
+    assert got[0] == ["1"] * 6, got
+    assert got[1][0] == "0", got
