@@ -329,6 +329,14 @@ void conv_stream_tile(aih::ConvStreamArgs *a, int32_t dt, aih::ConvStreamShape *
 // Whether the kernel's grid fits a launch.
 bool conv_stream_grid_ok(const aih::ConvStreamArgs &a) { return (uint64_t)a.mtiles * a.ntiles <= 0x7fffffffull; }
 
+// The plan of a call on it: in a direct kernel's place the tile of a wavefront,
+// as for those.
+aih_plan conv_stream_plan(const aih::ConvStreamArgs &a, const aih::ConvStreamShape &s, bool direct, size_t ws) {
+  const uint32_t grid = a.mtiles * a.ntiles;
+  if (direct) return aih_plan{AIH_VAR_DIRECT, 1, 32 * s.tm, 32 * s.tn, grid, ws};
+  return aih_plan{AIH_VAR_TILE, 1, aih::conv_stream_bm(s), aih::conv_stream_bn(s), grid, ws};
+}
+
 // The split factor of a pointwise call: the descriptor's, else (AUTO only)
 // the AIH_PW_SPLITK override, else 0 (the policy decides).
 int32_t pw_splitk_of(const aih_pw_desc *d) {
@@ -396,10 +404,7 @@ int plan_pw(const aih_pw_desc *d, GemmPlan *g) {
 //   below both, 32 -> 16 at 40x72 b64: 6.0 us there, 7.0 here).
 //   fp32: what the tiled GEMM ran with K whole (128 -> 320 at 20x36 b64: 74
 //   -> 43 us); calls it splits keep the split's shorter sums.
-// need: the workspace the call is checked against, the tiled GEMM's where
-// that is the base route (also for calls that run here without one).
-bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::ConvStreamShape *shape, size_t *need) {
-  *need = 0;
+bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::ConvStreamShape *shape) {
   const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;
   if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || d->dt != d->wdt || d->kg % ku || d->kg / ku < 4)
     return false;
@@ -413,7 +418,6 @@ bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::Co
   } else if (base == PW_TILED) {
     GemmPlan g;
     if (plan_pw(d, &g) || (d->dt == AIH_F32 && g.nsplit > 1)) return false;
-    *need = g.ws;
   } else {
     return false;
   }
@@ -445,14 +449,11 @@ size_t pw_ws(const aih_pw_desc *d, int base) {
 // kPwSplitkMaxM pixels and 24 of its 16-pixel x 16-channel blocks a CU (fp32 48
 // -> 192 at 10x18, 144 blocks: 6.4 us tiled, 2.7 here; 32 -> 960 at 1440
 // pixels, 5400: 7.0, 5.4; f16 48 -> 192 4.9, 2.6; 32 -> 960 at 1984 pixels,
-// 7440: 5.1, 5.0). The workspace is still the tiled GEMM's plan: a call without
-// it goes there and is refused.
-bool pw_short_k(const aih_pw_desc *d, const void *ws, size_t ws_bytes) {
+// 7440: 5.1, 5.0).
+bool pw_short_k(const aih_pw_desc *d) {
   if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || !pw_splitk_shape(d)) return false;
   const uint64_t M = (uint64_t)d->n * d->m;
-  if ((M + 15) / 16 * (d->ng / 4) > 24ull * aih::device_cus()) return false;
-  GemmPlan g;
-  return !plan_pw(d, &g) && (g.ws == 0 || (ws && ws_bytes >= g.ws && reinterpret_cast<uintptr_t>(ws) % 16 == 0));
+  return (M + 15) / 16 * (d->ng / 4) <= 24ull * aih::device_cus();
 }
 
 // Arguments of the one-dispatch split-K kernel and its K chunks (waves).
@@ -475,6 +476,32 @@ aih::PwSplitkArgs pw_splitk_args(const aih_pw_desc *d, uint32_t *waves) {
   a.has_res = d->residual ? 1 : 0;
   a.nxcd = aih::device_xcds();
   return a;
+}
+
+// What a pointwise call launches: its base route's kernel, or one that stands
+// in for it. ws is the tiled GEMM's workspace where that is the base route;
+// the call is refused without it whichever kernel runs.
+enum { PW_BASE = 0, PW_DMA = 1, PW_SHORT_K = 2 };
+struct PwLaunch {
+  int base, kernel;
+  size_t ws;
+  aih::ConvStreamArgs dma;
+  aih::ConvStreamShape dma_shape;
+};
+
+void pw_launch(const aih_pw_desc *d, PwLaunch *p) {
+  p->base = pw_base_route(d);
+  p->ws = pw_ws(d, p->base);
+  p->kernel = PW_BASE;
+  if (pw_dma_plan(d, p->base, &p->dma, &p->dma_shape))
+    p->kernel = PW_DMA;
+  else if (p->base == PW_TILED && pw_short_k(d))
+    p->kernel = PW_SHORT_K;
+}
+
+// A workspace as a plan asks for it.
+bool ws_fits(const void *ws, size_t bytes, size_t need) {
+  return need == 0 || (ws && bytes >= need && reinterpret_cast<uintptr_t>(ws) % 16 == 0);
 }
 
 int run_gemm(aih::GemmArgs &a, const GemmPlan &g, int32_t dt, int32_t wdt, bool igemm, bool pair, void *ws,
@@ -790,6 +817,34 @@ bool igemm_ksplit_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::C
   return true;
 }
 
+// What a KxK call (not the stem) launches: the direct or the tiled kernel of
+// its route, or one that stands in for it. The workspace is the tiled GEMM's
+// plan for what is not the direct kernel's route; the call is refused without
+// it whichever kernel runs.
+enum { IG_TILED = 0, IG_DIRECT = 1, IG_KSPLIT = 2, IG_STREAM = 3 };
+struct IgLaunch {
+  bool direct;
+  int kernel;
+  GemmPlan g;  // of a route that is not the direct kernel's
+  aih::IgDirectArgs da;
+  aih::ConvKsplitArgs ka;
+  aih::ConvStreamArgs sa;
+  aih::ConvStreamShape shape;
+};
+
+int igemm_launch(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, IgLaunch *p) {
+  p->g = GemmPlan{};
+  p->direct = ig_direct_plan(d, oh, ow, &p->da);
+  if (!p->direct && plan_igemm(d, &p->g)) return AIH_ERR;
+  if (igemm_ksplit_plan(d, oh, ow, &p->ka))
+    p->kernel = IG_KSPLIT;
+  else if (igemm_stream_plan(d, oh, ow, p->direct, p->g.nsplit == 1, &p->sa, &p->shape))
+    p->kernel = IG_STREAM;
+  else
+    p->kernel = p->direct ? IG_DIRECT : IG_TILED;
+  return AIH_OK;
+}
+
 // ---------------------------------------------------------------- fused inverted-residual block
 
 int check_ir(const aih_ir_block_desc *d, uint32_t *oh, uint32_t *ow) {
@@ -958,19 +1013,13 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out) {
     if (check_pw(d)) return AIH_ERR;
     if (!out) return fail("null plan");
     const uint64_t M = (uint64_t)d->n * d->m;
-    const int base = pw_base_route(d);
-    aih::ConvStreamArgs ca;
-    aih::ConvStreamShape cs;
-    size_t need;
-    if (pw_dma_plan(d, base, &ca, &cs, &need)) {
-      // what a direct kernel would take (up to 64 outputs) is reported as its
-      // 32 pixels a wavefront, the rest as the workgroup's tile
-      const uint32_t grid = ca.mtiles * ca.ntiles;
-      *out = base == PW_TILED ? aih_plan{AIH_VAR_TILE, 1, aih::conv_stream_bm(cs), aih::conv_stream_bn(cs), grid, need}
-                              : aih_plan{AIH_VAR_DIRECT, 1, 32, ca.N4 <= 32 ? 32u : 64u, grid, 0};
+    PwLaunch p;
+    pw_launch(d, &p);
+    if (p.kernel == PW_DMA) {
+      *out = conv_stream_plan(p.dma, p.dma_shape, p.base != PW_TILED, p.ws);
       return AIH_OK;
     }
-    switch (base) {
+    switch (p.kernel == PW_SHORT_K ? PW_SPLITK : p.base) {
       case PW_ROWS: {
         // pw_narrow_group(kg) lanes per pixel: 256 / that many pixels per workgroup
         const uint32_t ppb = 256 / aih::pw_narrow_group(d->kg);
@@ -982,7 +1031,7 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out) {
         // wavefronts (one wavefront: K whole, reported as a direct launch)
         uint32_t waves;
         const aih::PwSplitkArgs a = pw_splitk_args(d, &waves);
-        *out = aih_plan{waves > 1 ? AIH_VAR_SPLITK : AIH_VAR_DIRECT, waves, 16, 16, a.mblk * a.nblk, 0};
+        *out = aih_plan{waves > 1 ? AIH_VAR_SPLITK : AIH_VAR_DIRECT, waves, 16, 16, a.mblk * a.nblk, p.ws};
         return AIH_OK;
       }
       case PW_LDS: {
@@ -1026,22 +1075,22 @@ int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *
     if ((d->residual != 0) != (res != nullptr)) return fail("pw: res must be given iff residual");
     if (!aligned(x, 16) || !aligned(w, 16) || !aligned(y, 16) || !aligned(bias, 8) || (res && !aligned(res, 16)))
       return fail("pw: misaligned buffer (x, w, y, res need 16 bytes, bias 8)");
-    const int route = pw_base_route(d);
-    aih::ConvStreamArgs ca;
-    aih::ConvStreamShape cs;
-    size_t need;
-    if (pw_dma_plan(d, route, &ca, &cs, &need) && (need == 0 || (ws && ws_bytes >= need && aligned(ws, 16)))) {
-      // both operands streamed through LDS by DMA (a workspace too small for
-      // the plan is refused below, by the tiled GEMM)
-      ca.x = x;
-      ca.w = w;
-      ca.bias = bias;
-      ca.res = res;
-      ca.y = y;
-      const hipError_t e = aih::launch_conv_stream(ca, d->dt, cs, static_cast<hipStream_t>(stream));
+    PwLaunch p;
+    pw_launch(d, &p);
+    const int route = p.base;
+    // without the plan's workspace: on to the tiled GEMM, which refuses the call
+    const int kernel = ws_fits(ws, ws_bytes, p.ws) ? p.kernel : PW_BASE;
+    if (kernel == PW_DMA) {
+      // both operands streamed through LDS by DMA
+      p.dma.x = x;
+      p.dma.w = w;
+      p.dma.bias = bias;
+      p.dma.res = res;
+      p.dma.y = y;
+      const hipError_t e = aih::launch_conv_stream(p.dma, d->dt, p.dma_shape, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("pw stream launch: ") + hipGetErrorString(e));
     }
-    if (route == PW_SPLITK || (route == PW_TILED && pw_short_k(d, ws, ws_bytes))) {
+    if (route == PW_SPLITK || kernel == PW_SHORT_K) {
       // small M: K split across the wavefronts of one workgroup, reduced in
       // LDS, one dispatch, no workspace
       uint32_t waves;
@@ -1143,25 +1192,26 @@ int aih_conv_igemm_plan(const aih_igemm_desc *d, aih_plan *out) {
       *out = aih_plan{AIH_VAR_DIRECT, 1, 32, d->cout, grid, 0};
       return AIH_OK;
     }
-    aih::IgDirectArgs da;
-    if (ig_direct_plan(d, oh, ow, &da)) {
-      // few pixels or whole 64-channel taps: the LDS-streamed kernel in the
-      // direct one's place, reported as the direct route
-      aih::ConvStreamArgs sa;
-      aih::ConvStreamShape sh;
-      uint32_t grid = aih::ig_direct_grid(da.nblk, da.nj, da.N4);
-      if (igemm_stream_plan(d, oh, ow, true, true, &sa, &sh)) grid = sa.mtiles * sa.ntiles;
-      *out = aih_plan{AIH_VAR_DIRECT, 1, 32, da.N4 <= 32 ? 32u : 64u, grid, 0};
-      return AIH_OK;
+    IgLaunch p;
+    if (igemm_launch(d, oh, ow, &p)) return AIH_ERR;
+    // the variant is the route's; the split, the tile and the grid are the launch's
+    const int32_t whole = p.direct ? AIH_VAR_DIRECT : AIH_VAR_TILE;
+    switch (p.kernel) {
+      case IG_KSPLIT: {
+        const uint32_t chunks = div_ceil(p.ka.items, p.ka.per);
+        *out = aih_plan{!p.direct && chunks > 1 ? AIH_VAR_SPLITK : whole, chunks, 16, 16,
+                        (p.ka.M + 15) / 16 * p.ka.nblk, p.g.ws};
+        break;
+      }
+      case IG_STREAM:
+        *out = conv_stream_plan(p.sa, p.shape, p.direct, p.g.ws);
+        break;
+      case IG_DIRECT:
+        *out = aih_plan{whole, 1, 32, p.da.N4 <= 32 ? 32u : 64u, aih::ig_direct_grid(p.da.nblk, p.da.nj, p.da.N4), 0};
+        break;
+      default:
+        fill_plan(p.g, out);
     }
-    GemmPlan g;
-    if (plan_igemm(d, &g)) return AIH_ERR;
-    aih::ConvStreamArgs sa;
-    aih::ConvStreamShape sh;
-    if (igemm_stream_plan(d, oh, ow, false, g.nsplit == 1, &sa, &sh))
-      *out = aih_plan{AIH_VAR_TILE, 1, aih::conv_stream_bm(sh), aih::conv_stream_bn(sh), sa.mtiles * sa.ntiles, g.ws};
-    else
-      fill_plan(g, out);
     return AIH_OK;
   });
 }
@@ -1194,38 +1244,33 @@ int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const voi
       const hipError_t e = aih::launch_conv_stem(sa, d->dt, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("conv stem launch: ") + hipGetErrorString(e));
     }
-    // the workspace contract is the tiled GEMM's plan for what the direct
-    // kernel does not take: a call without it is refused there
-    aih::IgDirectArgs da;
-    const bool direct = ig_direct_plan(d, oh, ow, &da);
-    GemmPlan g{};
-    if (!direct && plan_igemm(d, &g)) return AIH_ERR;
-    const bool ws_ok = direct || g.ws == 0 || (ws && ws_bytes >= g.ws && aligned(ws, 16));
-    aih::ConvKsplitArgs ka;
-    if (ws_ok && igemm_ksplit_plan(d, oh, ow, &ka)) {
+    IgLaunch p;
+    if (igemm_launch(d, oh, ow, &p)) return AIH_ERR;
+    // without the plan's workspace: on to the tiled GEMM, which refuses the call
+    const int kernel = ws_fits(ws, ws_bytes, p.g.ws) ? p.kernel : IG_TILED;
+    if (kernel == IG_KSPLIT) {
       // few pixels: K over a workgroup's wavefronts
-      for (uint32_t i = 0; i < nin; ++i) ka.src[i] = inputs[i];
-      if (nin == 1) ka.src[1] = ka.src[0];
-      ka.w = w;
-      ka.bias = bias;
-      ka.res = res;
-      ka.y = y;
-      const hipError_t e = aih::launch_conv_ksplit(ka, d->dt, static_cast<hipStream_t>(stream));
+      for (uint32_t i = 0; i < nin; ++i) p.ka.src[i] = inputs[i];
+      if (nin == 1) p.ka.src[1] = p.ka.src[0];
+      p.ka.w = w;
+      p.ka.bias = bias;
+      p.ka.res = res;
+      p.ka.y = y;
+      const hipError_t e = aih::launch_conv_ksplit(p.ka, d->dt, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("igemm ksplit launch: ") + hipGetErrorString(e));
     }
-    aih::ConvStreamArgs ca;
-    aih::ConvStreamShape sh;
-    if (ws_ok && igemm_stream_plan(d, oh, ow, direct, g.nsplit == 1, &ca, &sh)) {
+    if (kernel == IG_STREAM) {
       // both operands streamed through LDS by DMA
-      ca.x = inputs[0];
-      ca.w = w;
-      ca.bias = bias;
-      ca.res = res;
-      ca.y = y;
-      const hipError_t e = aih::launch_conv_stream(ca, d->dt, sh, static_cast<hipStream_t>(stream));
+      p.sa.x = inputs[0];
+      p.sa.w = w;
+      p.sa.bias = bias;
+      p.sa.res = res;
+      p.sa.y = y;
+      const hipError_t e = aih::launch_conv_stream(p.sa, d->dt, p.shape, static_cast<hipStream_t>(stream));
       return e == hipSuccess ? AIH_OK : fail(std::string("igemm stream launch: ") + hipGetErrorString(e));
     }
-    if (direct) {
+    if (kernel == IG_DIRECT) {
+      aih::IgDirectArgs &da = p.da;
       // 3x3 with at most 64 output channels: weights resident in LDS,
       // activations straight into MFMA registers, no barriers after the load
       for (uint32_t i = 0; i < (d->nsrcs ? d->nsrcs : 1); ++i) da.src[i] = inputs[i];
@@ -1280,7 +1325,7 @@ int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const voi
     bool pair = d->dt != AIH_F32 && kg % 2 == 0;
     for (uint32_t i = 0; i < a.nparts; ++i)
       pair = pair && a.part_kg[i] % 2 == 0 && a.stride_kg[i] % 2 == 0 && a.off_kg[i] % 2 == 0;
-    return run_gemm(a, g, d->dt, d->wdt, true, pair, ws, ws_bytes, static_cast<hipStream_t>(stream));
+    return run_gemm(a, p.g, d->dt, d->wdt, true, pair, ws, ws_bytes, static_cast<hipStream_t>(stream));
   });
 }
 

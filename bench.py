@@ -405,15 +405,19 @@ def kernel_key(conv, op, n, dt, dtname) -> str:
         return f"pw_narrow_kernel<{dtname}>"
     if Lr.k == 1:
         p = conv.GemmPwSpec(m=Lr.ih * Lr.iw, kg=-(-Lr.cin // 4), ng=-(-Lr.cout // 4), dt=dt, n=n).plan()
-        if p.variant == conv.Variant.DIRECT:
-            return f"pw_direct_kernel<{dtname}>"
-        if p.variant == conv.Variant.SPLITK and p.bm == 16:
+        if p.bm == 16:
             return f"pw_splitk_kernel<{dtname}, {p.splitk}>"
+        direct = f"pw_direct_kernel<{dtname}>"
     else:
         p = conv.ConvIgemmSpec(ih=Lr.ih, iw=Lr.iw, cin=Lr.cin, cout=Lr.cout, k=Lr.k, s=Lr.s, pad=(Lr.pad,) * 4,
                                dt=dt, n=n).plan()
-        if p.variant == conv.Variant.DIRECT:
-            return f"conv_stem_kernel<{dtname}>" if Lr.cin <= 3 else f"conv_igemm_direct_kernel<{dtname}>"
+        if p.bm == 16:
+            return f"conv_ksplit_kernel<{dtname}>"
+        direct = f"conv_stem_kernel<{dtname}>" if Lr.cin <= 3 else f"conv_igemm_direct_kernel<{dtname}>"
+    oh, ow = Lr.out_hw()
+    streamed = p.bm == 64 or (Lr.cin > 3 and p.grid == -(-n * oh * ow // 64) * -(-Lr.cout // 64))
+    if streamed or p.variant == conv.Variant.DIRECT:
+        return f"conv_stream_kernel<{dtname},{'igemm' if Lr.k > 1 else 'pw'}>" if streamed else direct
     key = f"conv_gemm_kernel<{dtname},{dtname},BN={p.bn},{'igemm' if Lr.k > 1 else 'pw'}>"
     return key + ("+splitk_reduce" if p.splitk > 1 else "")
 

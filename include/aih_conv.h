@@ -154,12 +154,15 @@ typedef struct {
   uint32_t kg_pad;
 } aih_conv_desc;
 
-/* What a plan function chose; grid is the number of workgroups of the main kernel. */
+/* What a plan function chose: the route, the workspace that the call is
+ * checked for, and the launch -- splitk, bm, bn and grid are those of the kernel
+ * that runs, which may be one standing in for the route's own (aih_conv_pw and
+ * aih_conv_igemm below). */
 typedef struct {
-  int32_t variant;  /* AIH_VAR_TILE, AIH_VAR_SPLITK, AIH_VAR_ROWS or AIH_VAR_DIRECT */
-  uint32_t splitk;  /* K chunks (1 for TILE) */
-  uint32_t bm, bn;  /* output tile: pixels x channels */
-  uint32_t grid;
+  int32_t variant;  /* AIH_VAR_ROWS, AIH_VAR_DIRECT, else AIH_VAR_TILE (K whole) or AIH_VAR_SPLITK */
+  uint32_t splitk;  /* K chunks (1: K whole) */
+  uint32_t bm, bn;  /* output tile of a workgroup (AIH_VAR_DIRECT: of a wavefront): pixels x channels */
+  uint32_t grid;    /* workgroups of the main kernel */
   size_t ws_bytes;  /* workspace the call needs */
 } aih_plan;
 
@@ -230,15 +233,15 @@ typedef struct {
  * (32 pixels per wavefront, operands from memory into registers); fp32 with
  * at least 256 input channels and enough pixels for eight 32 x 32 wavefront
  * units per CU runs a GEMM whose operands stream through LDS by DMA over
- * the whole K (reported as AIH_VAR_TILE with bm = 96, no workspace). With
- * dt == wdt, whole 16-byte units (4 fp32 / 8 16-bit channels) a pixel, at
- * least 4 of them, and more than 2048 pixels, a GEMM with both operands
- * streamed through LDS runs at 16 bit what the tiled GEMM and most of what
- * the direct kernel would (the latter still reported as AIH_VAR_DIRECT, 32
- * pixels a wavefront), and at fp32 what the tiled GEMM would with K whole; and
- * up to 2048 pixels the split-K kernel runs the tiled GEMM's calls of few
- * 16 x 16 output blocks. The plan is still the tiled GEMM's for both, its
- * workspace too, and a call without it is refused. */
+ * the whole K (reported as AIH_VAR_TILE with bm = 96, no workspace). Two
+ * kernels stand in for others with dt == wdt: beyond 2048 pixels of whole
+ * 16-byte units (4 fp32 / 8 16-bit channels), at least 4 of them, a GEMM with
+ * both operands streamed through LDS runs at 16 bit what the tiled GEMM and
+ * most of what the direct kernel would, and at fp32 what the tiled GEMM would
+ * with K whole; and up to 2048 pixels the split-K kernel (bm = bn = 16) runs
+ * the tiled GEMM's calls of few 16 x 16 output blocks. The workspace stays
+ * the one of the kernel they stand in for (neither uses it), and a call
+ * without it is refused. */
 int aih_conv_pw(const aih_pw_desc *d, const void *x, const void *w, const void *bias,
                 const void *res, void *y, void *ws, size_t ws_bytes, aih_stream stream);
 int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);
@@ -248,11 +251,13 @@ int aih_conv_pw_plan(const aih_pw_desc *d, aih_plan *out);
  * over at most 3 input channels with cout 32 or 64, AIH_VAR_AUTO, splitk 0 and
  * dt == wdt -- the stem -- runs a dedicated kernel (all 27 tap-channel values
  * in one MFMA operand) instead of the planned implicit GEMM; it needs no
- * workspace. Other one-input AIH_VAR_AUTO calls with dt == wdt and whole
- * 16-byte units may run a GEMM with both operands streamed through LDS in the
- * place of the tiled GEMM or of the direct 3x3 kernel, and ones of at most two
- * inputs and few pixels a kernel whose workgroups split K on chip; the plan
- * reports the route and the workspace of the kernel they stand in for. */
+ * workspace. Two kernels stand in for others in AIH_VAR_AUTO calls with splitk
+ * 0, dt == wdt and whole 16-byte units: a GEMM with both operands streamed
+ * through LDS (one input) for the tiled GEMM or the direct 3x3 kernel, and for
+ * few pixels of at most two inputs one whose workgroups split K on chip (bm =
+ * bn = 16). In the direct kernel's place they are reported as AIH_VAR_DIRECT;
+ * the workspace stays the one of the kernel they stand in for (neither uses
+ * it), and a call without it is refused. */
 int aih_conv_igemm(const aih_igemm_desc *d, const void *const *inputs, const void *w,
                    const void *bias, const void *res, void *y, void *ws, size_t ws_bytes,
                    aih_stream stream);

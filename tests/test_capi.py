@@ -432,6 +432,56 @@ def test_env_overrides_of_the_split_policy():
     assert int(_plan_in_subprocess({"AIH_IGEMM_NO_SPLIT": "1"}, IG_SPLIT_PROBE)) == 1
 
 
+def test_plans_report_the_kernel_that_runs():
+    """The tile, the split and the grid of a plan are the launch's, on both
+    sides of each limit between kernels (256 CUs); the direct route and the
+    workspace stay those of the kernel a launch stands in for. (The streamed
+    GEMM in a direct kernel's place: 64 x 64 tiles of four wavefronts.)"""
+    V, D = conv.Variant, conv.DType
+    DIRECT, TILE, SPLITK = V.DIRECT, V.TILE, V.SPLITK
+
+    def pw(m, cin, cout, dt, n=1):
+        p = conv.GemmPwSpec(m=m, kg=cin // 4, ng=cout // 4, n=n, dt=dt).plan()
+        return p.variant, p.splitk, p.bm, p.bn, p.grid
+
+    # LDS-streamed GEMM: beyond 2048 pixels (the split-K kernel up to there)
+    assert pw(2048, 192, 320, D.F16) == (SPLITK, 2, 16, 16, 128 * 20)
+    assert pw(2049, 192, 320, D.F16) == (TILE, 1, 64, 64, 33 * 5)
+    assert pw(2049, 28, 320, D.F16)[2] == 128  # 4-channel groups that are not whole 16-byte units
+    assert pw(2049, 24, 320, D.F16)[2] == 128  # three units
+    assert pw(2049, 32, 320, D.F16)[2] == 64
+    # in the direct kernel's place: more than 32 outputs, or 64 channels
+    assert pw(65536, 32, 32, D.F16) == (DIRECT, 1, 32, 32, 512)
+    assert pw(65536, 32, 36, D.F16) == (DIRECT, 1, 32, 32, 1024)
+    assert pw(65536, 64, 32, D.F16) == (DIRECT, 1, 32, 32, 1024)
+    # short K over 16 x 16 blocks: at most 24 of them a CU
+    assert pw(2048, 48, 768, D.F32) == (DIRECT, 1, 16, 16, 128 * 48)
+    assert pw(2048, 48, 784, D.F32)[2] == 128
+
+    def ig(dt, **kw):
+        p = conv.ConvIgemmSpec(**{**dict(ih=64, iw=64, cin=64, cout=64, k=3, pad=(1, 1, 1, 1), dt=dt), **kw}).plan()
+        return p.variant, p.splitk, p.bm, p.bn, p.grid, p.ws_bytes > 0
+
+    # K over the wavefronts: four (fp32) or two (16 bit) 16 x 16 blocks a CU
+    assert ig(D.F32) == (DIRECT, 9, 16, 16, 1024, False)
+    assert ig(D.F32, iw=65) == (DIRECT, 1, 32, 32, 65, False)
+    assert ig(D.F16, ih=32) == (DIRECT, 9, 16, 16, 512, False)
+    assert ig(D.F16, ih=33) == (DIRECT, 1, 32, 32, 33, False)
+    assert ig(D.F32, ih=9, iw=16, cin=240, cout=96) == (SPLITK, 9, 16, 16, 54, True)
+    assert ig(D.F32, ih=9, iw=16, k=1, pad=(0,) * 4) == (SPLITK, 4, 16, 16, 36, True)  # 4 steps: 4 wavefronts
+    assert ig(D.F16, ih=9, iw=16, cin=28, cout=96)[2] == 128  # not whole 16-byte units
+    # the direct kernel from 65536 pixels, 16-bit calls of whole 64-channel taps aside
+    assert ig(D.F32, n=15) == (DIRECT, 1, 32, 32, 960, False) and ig(D.F32, n=16) == (DIRECT, 1, 32, 64, 256, False)
+    assert ig(D.F16, n=16) == (DIRECT, 1, 32, 32, 1024, False)
+    assert ig(D.F16, n=16, cin=72) == (DIRECT, 1, 32, 64, 256, False)
+    two = dict(cin=72, srcs=[conv.SrcView(c=48), conv.SrcView(c=24)], cout=32)
+    assert ig(D.F16, ih=65, **two) == (DIRECT, 1, 32, 32, 17, False)
+    # in the tiled GEMM's place: fp32 with K whole, 16 bit from 48 tiles of 64 x 64
+    assert ig(D.F32, cout=128, n=20) == (TILE, 1, 128, 128, 640, False)
+    assert ig(D.F16, ih=24, cout=128) == (TILE, 1, 64, 64, 48, True)
+    assert ig(D.F16, ih=23, cout=128)[2] == 128
+
+
 def test_ir_block_forced_weight_placement():
     base = dict(ih=40, iw=72, cin=64, cexp=256, cout=64, s=1, n=64, dt=conv.DType.F16)
     for tile in [(0, 0), (8, 8), (4, 16)]:

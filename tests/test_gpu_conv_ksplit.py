@@ -43,11 +43,18 @@ def check(name, err, dt):
     assert err <= BAR[dt], (name, err)
 
 
+CUS = torch.cuda.get_device_properties(0).multi_processor_count
+
+
 @pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "x".join(map(str, c[:7])))
 def test_igemm(case, dt):
     ih, iw, cin, cout, k, s, d, pad, act, res, n = case
     r = G.run_igemm(ih, iw, cin, cout, k, s, pad, act, res, dt, 9700 + cin, n=n, d=d)
+    oh, ow = G.orc.out_hw(G.orc.conv2d(cin, cout, k=k, s=s, pad=list(pad), dil=d), ih, iw)
+    blocks = -(-n * oh * ow // 16) * -(-cout // 16)
+    here = blocks <= CUS * (4 if dt == F32 else 2) and (dt == F32 or cin % 8 == 0)
+    assert ((r.plan.bm, r.plan.bn, r.plan.grid) == (16, 16, blocks)) == here, (blocks, r.plan)
     assert not np.isnan(np.asarray(r.got)).any(), case
     check(f"igemm {case}", G.rel_err(r.got, r.want_r), dt)
 
@@ -63,6 +70,7 @@ PW = [(1, 1, 4, 80, 1), (10, 18, 48, 192, 1), (7, 5, 44, 144, 3), (23, 31, 60, 1
 def test_pointwise_short_k(case, dt):
     h, w, cin, cout, n = case
     r = G.run_pw(h, w, cin, cout, "relu6", True, dt, 9850 + cin, n=n)
+    assert ((r.plan.bm, r.plan.bn) == (16, 16)) == (-(-n * h * w // 16) * (cout // 16) <= 24 * CUS), r.plan
     assert not np.isnan(np.asarray(r.got)).any(), case
     check(f"pw {case} {r.plan}", G.rel_err(r.got, r.want_r), dt)
 
@@ -79,6 +87,7 @@ def test_two_parts(dt):
     spec = G.conv.ConvIgemmSpec(ih=ih, iw=iw, cin=c0 + c1, cout=cout, k=3, pad=(1, 1, 1, 1), act=G.ACT["relu"],
                                 dt=G.conv.DType(dt), srcs=[G.conv.SrcView(c=c0, stride_c=40, c_off=8),
                                                            G.conv.SrcView(c=c1, stride_c=c1, c_off=0)])
+    assert spec.plan().bm == 16
     yd = G.poisoned(ih * iw * cout, dt)
     spec.run([G.dev(G.orc.pack_nhwc(xa, 1, ih, iw, 40, dt)), G.dev(G.orc.pack_nhwc(xb, 1, ih, iw, c1, dt))], G.dev(wp),
              G.dev(G.orc.pack_bias(b, cout, dt)), None, yd)
@@ -95,6 +104,7 @@ def test_infinities_stay_in_their_taps():
     x = torch.from_numpy(rng.standard_normal((1, h, w, c)).astype(np.float32)).cuda()
     x[0, 0, 0] = float("inf")
     op = G.conv.ConvOp(ih=h, iw=w, cin=c, cout=cout, kh=3, kw=3, pad=(1,) * 4)
+    assert op.plan().bm == 16
     p, _ = G.conv.pack_weights_conv(wts.ravel(), cout, c, 3, 3, 4, G.conv.DType.F32)
     b = G.conv.pack_bias(np.zeros(cout, np.float32), cout, G.conv.DType.F32)
     y = torch.full((1, h, w, cout), float("nan"), device="cuda")

@@ -28,8 +28,8 @@ def check(name, r, dt):
     assert err <= BAR[dt], (name, err)
 
 
-# (h, w, cin, cout, n), act, residual, (bm, bn) of the 16-bit plan (None: the
-# direct route's, at most 64 outputs)
+# (h, w, cin, cout, n), act, residual, (bm, bn) of the 16-bit plan (None: 64 x 64
+# in the place of a direct kernel, at most 64 outputs)
 PW = [((23, 37, 32, 96, 3), "relu", False, (64, 64)),        # one unit a lane half, 40 pixels in the last tile
       ((21, 37, 72, 100, 3), "hardswish", True, (64, 64)),   # K ends inside a stage; 8-byte output rows
       ((24, 30, 328, 132, 3), "relu6", True, (64, 64)),      # stages of 8 units, 41 units
@@ -50,6 +50,7 @@ def test_pointwise(case, dt):
         assert (r.plan.variant, r.plan.bm, r.plan.bn) == (V.TILE, *tile), r.plan
     elif dt != F32:
         assert r.plan.variant == V.DIRECT and r.plan.ws_bytes == 0, r.plan
+        assert r.plan.grid == -(-n * h * w // 64), r.plan
     check(f"pw {case}", r, dt)
 
 
@@ -58,19 +59,33 @@ IG = [(23, 31, 64, 100, 3, 1, 1, (1, 1, 1, 1), "relu", True, 5),
       (41, 37, 32, 96, 3, 2, 1, (0, 1, 1, 0), "hardswish", False, 6),      # 4 units a tap: a stage is a tap
       (40, 50, 40, 72, 5, 1, 1, (2, 2, 2, 2), "none", False, 2),           # 5 units a tap: stages cross taps
       (33, 47, 72, 68, 3, 1, 2, (2, 2, 2, 2), "relu6", True, 3),           # dilated
-      (30, 40, 36, 80, 2, 1, 1, (0, 0, 0, 0), "relu", False, 4),           # fp32 only: an odd kg count
+      (30, 40, 36, 80, 2, 1, 1, (0, 0, 0, 0), "relu", False, 4),           # an odd kg count, few pixels: the tiled GEMM
       (45, 83, 48, 128, 3, 1, 1, (1, 1, 1, 1), "relu", True, 18),          # 128 x 128 tiles, a ragged last one
       (45, 83, 32, 96, 3, 1, 1, (1, 1, 1, 1), "none", False, 18),          # 128 x 96
       (45, 83, 32, 176, 3, 2, 1, (1, 1, 1, 1), "relu", False, 60),         # 128 x 64
       (33, 47, 64, 64, 3, 1, 1, (1, 1, 1, 1), "relu", True, 11),           # in place of the direct kernel
-      (65, 64, 64, 36, 3, 1, 1, (1, 1, 1, 1), "relu", False, 17)]          # the same above 65536 pixels, 16 bit
+      (65, 64, 64, 36, 3, 1, 1, (1, 1, 1, 1), "relu", False, 17),          # the same above 65536 pixels, 16 bit
+      # fp32 only, odd kg counts: a K tail, stages that cross taps, dilated with a stride
+      (60, 80, 36, 80, 2, 1, 1, (0, 0, 0, 0), "relu", False, 10),
+      (45, 83, 20, 96, 5, 1, 1, (2, 2, 2, 2), "none", True, 18),
+      (45, 83, 36, 68, 3, 2, 2, (2, 2, 2, 2), "relu6", True, 60)]
+# their tiles at fp32 and at 16 bit (in the direct kernel's place a wavefront's);
+# None: another kernel runs the call (fp32 with a split K, a few pixels, an odd kg count)
+IG_TILES = [(None, (64, 64)), (None, (64, 64)), (None, (64, 64)), (None, (64, 64)), (None, None),
+            ((128, 128),) * 2, ((128, 96),) * 2, ((128, 64),) * 2, ((32, 32),) * 2, (None, (32, 32)),
+            ((64, 64), None), ((128, 96), None), ((64, 64), None)]
 
 
 @pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("case", IG, ids=lambda c: "x".join(map(str, c[:7])))
 def test_igemm(case, dt):
     ih, iw, cin, cout, k, s, d, pad, act, res, n = case
-    check(f"igemm {case}", G.run_igemm(ih, iw, cin, cout, k, s, pad, act, res, dt, 9300 + cin, n=n, d=d), dt)
+    r = G.run_igemm(ih, iw, cin, cout, k, s, pad, act, res, dt, 9300 + cin, n=n, d=d)
+    tile = IG_TILES[IG.index(case)][dt != F32]
+    if tile == (32, 32):
+        assert r.plan.grid == -(-n * ih * iw // 64), r.plan
+    assert ((r.plan.bm, r.plan.bn) == tile and r.plan.splitk == 1) if tile else r.plan.bm != 64, r.plan
+    check(f"igemm {case}", r, dt)
 
 
 # ih, iw, cin, cout, s, d, pad, n: 1x1 convs through the KxK entry, past the
@@ -88,7 +103,9 @@ ONE_TAP = [(97, 101, 64, 68, 2, 1, (0, 0, 0, 0), 5),
 @pytest.mark.parametrize("case", ONE_TAP, ids=lambda c: "x".join(map(str, c[:6])))
 def test_one_tap_with_stride_and_padding(case, dt):
     ih, iw, cin, cout, s, d, pad, n = case
-    check(f"1x1 {case}", G.run_igemm(ih, iw, cin, cout, 1, s, pad, "none", False, dt, 9350 + cin, n=n, d=d), dt)
+    r = G.run_igemm(ih, iw, cin, cout, 1, s, pad, "none", False, dt, 9350 + cin, n=n, d=d)
+    assert r.plan.bm == 64 or dt == F32, r.plan  # (fp32 sums the tiled GEMM splits stay there)
+    check(f"1x1 {case}", r, dt)
 
 
 @pytest.mark.parametrize("dt", [F32, F16], ids=["f32", "f16"])
