@@ -444,16 +444,26 @@ size_t pw_ws(const aih_pw_desc *d, int base) {
   return base == PW_TILED && !plan_pw(d, &g) ? g.ws : 0;
 }
 
-// A call of the tiled GEMM's (fewer than 64 input channels, more outputs than
-// the direct kernel holds) that the one-dispatch split-K kernel runs: at most
-// kPwSplitkMaxM pixels and 24 of its 16-pixel x 16-channel blocks a CU (fp32 48
-// -> 192 at 10x18, 144 blocks: 6.4 us tiled, 2.7 here; 32 -> 960 at 1440
-// pixels, 5400: 7.0, 5.4; f16 48 -> 192 4.9, 2.6; 32 -> 960 at 1984 pixels,
-// 7440: 5.1, 5.0).
+// A call of the tiled GEMM's that the one-dispatch split-K kernel runs, up to
+// kPwSplitkMaxM pixels. That kernel reuses nothing (each 16-pixel x 16-channel
+// block reads its rows of both operands), so it takes few blocks and a short K
+// (us tiled / here, blocks):
+//   fewer than 64 input channels, 24 blocks a CU: fp32 48 -> 192 at 180 pixels
+//   6.4 / 2.7 (144), 32 -> 960 at 1440 7.0 / 5.4 (5400); f16 48 -> 192 4.9 /
+//   2.6, 32 -> 960 at 1984 5.1 / 5.0 (7440).
+//   up to 320, 24 a CU, at fp32 and where the tiled GEMM splits K: fp32 64 ->
+//   768 at 2048 10.3 / 8.8 (6144), 320 -> 768 35.4 / 25.9, 576 -> 768 44.7 /
+//   54.7; f16 192 -> 768 21.2 / 14.3, 320 -> 768 27.0 / 21.4, 576 -> 768
+//   28.5 / 35.7, 1280 -> 768 33.8 / 84.3.
+//   16 bit with K whole there: up to 96, 20 a CU: 64 -> 576 at 2048 6.2 / 5.9
+//   (4608), 64 -> 960 at 1440 6.3 / 6.6 (5400), 96 -> 576 7.1 / 6.1, 128 -> 576
+//   8.0 / 8.5.
 bool pw_short_k(const aih_pw_desc *d) {
-  if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || !pw_splitk_shape(d)) return false;
-  const uint64_t M = (uint64_t)d->n * d->m;
-  return (M + 15) / 16 * (d->ng / 4) <= 24ull * aih::device_cus();
+  if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || !pw_splitk_shape(d) || d->kg > 80) return false;
+  const uint64_t M = (uint64_t)d->n * d->m, blocks = (M + 15) / 16 * (d->ng / 4), cus = aih::device_cus();
+  GemmPlan g;
+  if (d->kg < 16 || d->dt == AIH_F32 || (!plan_pw(d, &g) && g.nsplit > 1)) return blocks <= 24 * cus;
+  return d->kg <= 24 && blocks <= 20 * cus;
 }
 
 // Arguments of the one-dispatch split-K kernel and its K chunks (waves).

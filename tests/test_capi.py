@@ -457,6 +457,14 @@ def test_plans_report_the_kernel_that_runs():
     # short K over 16 x 16 blocks: at most 24 of them a CU
     assert pw(2048, 48, 768, D.F32) == (DIRECT, 1, 16, 16, 128 * 48)
     assert pw(2048, 48, 784, D.F32)[2] == 128
+    # a longer K there: up to 320 channels at fp32 or where the tiled GEMM
+    # splits K, 96 (and 20 blocks a CU) where it does not; a long one never
+    for dt in (D.F32, D.F16, D.BF16):
+        assert pw(180, 960, 576, dt, n=10)[2] == 128
+        assert pw(1800, 320, 576, dt)[2] == 16 and pw(1800, 324, 576, dt)[2] == 128
+        assert pw(1800, 96, 576, dt)[2] == 16
+    assert pw(2048, 128, 768, D.F32)[2] == 16 and pw(2048, 128, 768, D.F16)[2] == 128
+    assert pw(2048, 64, 640, D.F16)[2] == 16 and pw(2048, 64, 656, D.F16)[2] == 128
 
     def ig(dt, **kw):
         p = conv.ConvIgemmSpec(**{**dict(ih=64, iw=64, cin=64, cout=64, k=3, pad=(1, 1, 1, 1), dt=dt), **kw}).plan()

@@ -75,6 +75,21 @@ def test_pointwise_short_k(case, dt):
     check(f"pw {case} {r.plan}", G.rel_err(r.got, r.want_r), dt)
 
 
+# h, w, cin, cout; on 16 x 16 blocks at fp32 and at 16 bit
+PW_LONGER = [((45, 40, 96, 576), (True, True)), ((45, 40, 320, 576), (True, True)),
+             ((45, 40, 324, 576), (False, False)), ((32, 64, 128, 768), (True, False))]
+
+
+@pytest.mark.skipif(CUS != 256, reason="the limits are multiples of the CUs")
+@pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", PW_LONGER, ids=lambda c: "x".join(map(str, c[0])))
+def test_pointwise_longer_k(case, dt):
+    (h, w, cin, cout), here = case
+    r = G.run_pw(h, w, cin, cout, "relu", False, dt, 9870 + cin)
+    assert (r.plan.bm == 16) == here[dt != F32], r.plan
+    check(f"pw {case[0]} {r.plan}", G.rel_err(r.got, r.want_r), dt)
+
+
 @pytest.mark.parametrize("dt", [F32, F16], ids=["f32", "f16"])
 def test_two_parts(dt):
     """A concat read: 24 channels of a 40-channel tensor, then 16 plain ones."""
