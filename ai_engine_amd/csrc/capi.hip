@@ -706,7 +706,12 @@ bool ig_direct_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::IgDi
 // whole.
 //   tiled calls at 16 bit: from 48 tiles of 64 x 64 (128 -> 128 3x3 at 40x72
 //   b32: 69.7 -> 41 us; fewer tiles, 256 -> 256 at 10x18 b4 is 48 of them:
-//   18.1 -> 15.8); at fp32 the unsplit ones (64 -> 128 b32: 222 -> 117 us;
+//   18.1 -> 15.8), below 100 of them, where the tiled GEMM splits K in 5 to 8,
+//   up to 72 products of K a tile and with the weights within an XCD's 4 MB L2
+//   (720 pixels, 256 outputs, 48 tiles: K = 3200 22.1 -> 21.6, 6400 33.9 ->
+//   38.8, 8640 41.8 -> 70.3; 1440 pixels, 92 tiles: 6400 49.2 -> 39.2, 12544
+//   91.2 -> 98.6; 512 outputs at 720 pixels, 96 tiles: 4032 35.1 -> 31.5, 4608
+//   38.6 -> 39.6); at fp32 the unsplit ones (64 -> 128 b32: 222 -> 117 us;
 //   split ones keep the split's shorter sums).
 //   direct calls below 65536 pixels, whose 32-pixel wavefronts leave CUs idle
 //   (64 -> 64 fp32 at 40x72 b4: 44 -> 17 us, f16 15.3 -> 6.6); at fp32 only
@@ -720,14 +725,16 @@ bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool d
   const uint32_t kg = div_ceil(d->cin, 4), n4 = div_ceil(d->cout, 4) * 4;
   const uint32_t stride = d->nsrcs ? d->srcs[0].stride_c / 4 : kg, off = d->nsrcs ? d->srcs[0].c_off / 4 : 0;
   if (kg % ku || stride % ku || off % ku || kg / ku < 4) return false;
-  const uint32_t M = d->n * oh * ow;
+  const uint32_t M = d->n * oh * ow, kgp = div_ceil(kg, 4) * 4;
+  const uint64_t tiles = (uint64_t)div_ceil(M, 64) * div_ceil(n4, 64);
+  const uint64_t wb = (uint64_t)d->k * d->k * kgp * n4 * 4 * es;
   if (direct) {
     if (M < 65536 ? d->dt == AIH_F32 && n4 <= 32 : d->dt == AIH_F32 || kg % 16) return false;
   } else {
-    if (d->dt == AIH_F32 ? !unsplit : (uint64_t)div_ceil(M, 64) * div_ceil(n4, 64) < 48) return false;
+    if (d->dt == AIH_F32 ? !unsplit : tiles < 48) return false;
+    if (tiles < 100 && (d->k * d->k * kg * 4ull > 72 * tiles || wb > 4u << 20) && !unsplit) return false;
   }
-  const uint32_t kgp = div_ceil(kg, 4) * 4;
-  const uint64_t xb = (uint64_t)d->n * d->ih * d->iw * stride * 4 * es, wb = (uint64_t)d->k * d->k * kgp * n4 * 4 * es;
+  const uint64_t xb = (uint64_t)d->n * d->ih * d->iw * stride * 4 * es;
   if (xb >= 0x80000000ull || wb >= 0x80000000ull) return false;
   std::memset(a, 0, sizeof(*a));
   a->x_bytes = (uint32_t)xb;

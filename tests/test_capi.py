@@ -488,6 +488,13 @@ def test_plans_report_the_kernel_that_runs():
     assert ig(D.F32, cout=128, n=20) == (TILE, 1, 128, 128, 640, False)
     assert ig(D.F16, ih=24, cout=128) == (TILE, 1, 64, 64, 48, True)
     assert ig(D.F16, ih=23, cout=128)[2] == 128
+    # below 100 tiles up to 72 products of K a tile, weights up to 4 MB
+    few = dict(ih=20, iw=36, cout=256)  # 48 tiles
+    assert ig(D.F16, **few, cin=256, k=5, pad=(2,) * 4)[2] == 128
+    assert ig(D.F16, **few, cin=384)[2] == 64 and ig(D.F16, **few, cin=392)[2] == 128
+    wide = dict(ih=20, iw=36, cout=512)  # 96
+    assert ig(D.F16, **wide, cin=448)[2] == 64 and ig(D.F16, **wide, cin=512)[2] == 128
+    assert ig(D.F16, ih=40, iw=40, cout=256, cin=256, k=7, pad=(3,) * 4)[2] == 64  # 100
 
 
 def test_ir_block_forced_weight_placement():
