@@ -400,8 +400,11 @@ int plan_pw(const aih_pw_desc *d, GemmPlan *g) {
 //   16 bit: what the tiled GEMM ran (192 -> 768 at 21x37 b64: 64.5 -> 35 us),
 //   and what the direct kernels ran with more than 32 outputs or at least 64
 //   channels, beyond 2048 pixels (32 -> 64 at 80x144 b64: 56.7 -> 35 us, 128
-//   -> 32 at 40x72 b64: 19.6 -> 12.6, 128 -> 64 at 11520 pixels 5.9 -> 3.5;
-//   below both, 32 -> 16 at 40x72 b64: 6.0 us there, 7.0 here).
+//   -> 32 at 40x72 b64: 19.6 -> 12.6; below both, 32 -> 16 at 40x72 b64: 6.0
+//   us there, 7.0 here). Launches of few 16x16 blocks stay (us there / here:
+//   64 -> 32 at 4096 pixels, 2 blocks a CU, 3.4 / 3.9, at 11520, 5.6, 3.9 /
+//   4.0, at 16384, 8, 4.3 / 4.0; 128 -> 32 at 5760, 2.8, 3.9 / 4.2, at 8192, 4,
+//   4.2 / 4.2, at 11520 4.7 / 4.3).
 //   fp32: what the tiled GEMM ran with K whole (128 -> 320 at 20x36 b64: 74
 //   -> 43 us); calls it splits keep the split's shorter sums.
 bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::ConvStreamShape *shape) {
@@ -413,8 +416,11 @@ bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::Co
   if (M <= aih::kPwSplitkMaxM || xb >= 0x80000000ull || wb >= 0x80000000ull) return false;
   if (base == PW_DIRECT || base == PW_LDS || base == PW_SPLITK) {
     if (d->dt == AIH_F32 || (N4 <= 32 && d->kg < 16)) return false;
-    // 16x16-block launches of a short K stay
-    if (base == PW_SPLITK && d->kg < 16) return false;
+    // 16x16-block launches (beyond 2048 pixels at most 128 channels) stay with
+    // a short K, and with few blocks: up to 6 a CU, 3 beyond 96 channels
+    if (base == PW_SPLITK &&
+        (d->kg < 16 || (M + 15) / 16 * (N4 / 16) <= (d->kg <= 24 ? 6ull : 3ull) * aih::device_cus()))
+      return false;
   } else if (base == PW_TILED) {
     GemmPlan g;
     if (plan_pw(d, &g) || (d->dt == AIH_F32 && g.nsplit > 1)) return false;

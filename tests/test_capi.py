@@ -454,6 +454,11 @@ def test_plans_report_the_kernel_that_runs():
     assert pw(65536, 32, 32, D.F16) == (DIRECT, 1, 32, 32, 512)
     assert pw(65536, 32, 36, D.F16) == (DIRECT, 1, 32, 32, 1024)
     assert pw(65536, 64, 32, D.F16) == (DIRECT, 1, 32, 32, 1024)
+    # few 16 x 16 blocks stay: six a CU up to 96 channels, three beyond
+    assert pw(12288, 64, 32, D.F16) == (DIRECT, 1, 16, 16, 1536)
+    assert pw(12289, 64, 32, D.F16) == (DIRECT, 1, 32, 32, 193)
+    assert pw(6144, 128, 32, D.F16) == (DIRECT, 1, 16, 16, 768)
+    assert pw(6145, 128, 32, D.F16) == (DIRECT, 1, 32, 32, 97)
     # short K over 16 x 16 blocks: at most 24 of them a CU
     assert pw(2048, 48, 768, D.F32) == (DIRECT, 1, 16, 16, 128 * 48)
     assert pw(2048, 48, 784, D.F32)[2] == 128
