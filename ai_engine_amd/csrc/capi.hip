@@ -721,9 +721,12 @@ bool ig_direct_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::IgDi
 //   split ones keep the split's shorter sums).
 //   direct calls below 65536 pixels, whose 32-pixel wavefronts leave CUs idle
 //   (64 -> 64 fp32 at 40x72 b4: 44 -> 17 us, f16 15.3 -> 6.6); at fp32 only
-//   with more than 32 outputs (72 -> 32 b8: 29.7 there, 30.1 here); at or
-//   above, 16-bit ones with whole 64-channel taps (64 -> 64 b32: 22.4 -> 17.8,
-//   128 -> 64 38.2 -> 28.8; 96 -> 64 22.6 there, 25.5 here).
+//   with more than 32 outputs (72 -> 32 b8: 29.7 there, 30.1 here), at 16 bit
+//   below 32768 pixels with at most 32 outputs and 128 channels, half of whose
+//   tile is padding (48 -> 24 at 23040 pixels 7.9 there, 8.1 here, at 46080 8.3
+//   and 9.4; 80 -> 32 10.8 and 9.4, 11.1 and 11.7; 160 -> 24 at 46080 20.0 and
+//   18.6); above, 16-bit ones with whole 64-channel taps (64 -> 64 b32: 22.4 ->
+//   17.8, 128 -> 64 38.2 -> 28.8; 96 -> 64 22.6 there, 25.5 here).
 bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool direct, bool unsplit,
                        aih::ConvStreamArgs *a, aih::ConvStreamShape *shape) {
   if (d->variant != AIH_VAR_AUTO || d->splitk != 0 || d->dt != d->wdt || d->nsrcs > 1) return false;
@@ -735,7 +738,8 @@ bool igemm_stream_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, bool d
   const uint64_t tiles = (uint64_t)div_ceil(M, 64) * div_ceil(n4, 64);
   const uint64_t wb = (uint64_t)d->k * d->k * kgp * n4 * 4 * es;
   if (direct) {
-    if (M < 65536 ? d->dt == AIH_F32 && n4 <= 32 : d->dt == AIH_F32 || kg % 16) return false;
+    const bool few = n4 <= 32 && kg <= 32;  // outputs and channels
+    if (M < (few ? 32768u : 65536u) ? d->dt == AIH_F32 && n4 <= 32 : d->dt == AIH_F32 || kg % 16) return false;
   } else {
     if (d->dt == AIH_F32 ? !unsplit : tiles < 48) return false;
     if (tiles < 100 && (d->k * d->k * kg * 4ull > 72 * tiles || wb > 4u << 20) && !unsplit) return false;

@@ -487,6 +487,10 @@ def test_plans_report_the_kernel_that_runs():
     assert ig(D.F32, n=15) == (DIRECT, 1, 32, 32, 960, False) and ig(D.F32, n=16) == (DIRECT, 1, 32, 64, 256, False)
     assert ig(D.F16, n=16) == (DIRECT, 1, 32, 32, 1024, False)
     assert ig(D.F16, n=16, cin=72) == (DIRECT, 1, 32, 64, 256, False)
+    # ... from 32768 at 16 bit with at most 32 outputs and 128 channels
+    assert ig(D.F16, cin=48, cout=24, n=7) == (DIRECT, 1, 32, 32, 448, False)
+    assert ig(D.F16, cin=48, cout=24, n=8) == (DIRECT, 1, 32, 32, 128, False)
+    assert ig(D.F16, cin=136, cout=24, n=8)[4] == ig(D.F16, cin=48, cout=36, n=8)[4] == 512
     two = dict(cin=72, srcs=[conv.SrcView(c=48), conv.SrcView(c=24)], cout=32)
     assert ig(D.F16, ih=65, **two) == (DIRECT, 1, 32, 32, 17, False)
     # in the tiled GEMM's place: fp32 with K whole, 16 bit from 48 tiles of 64 x 64
