@@ -101,8 +101,27 @@ using namespace aih;
 
 constexpr size_t kReadFloats = 16u << 20;
 
+// Makes `device` current while it lives.
+struct OnDevice {
+  int was = -1;
+  hipError_t e;
+  explicit OnDevice(int device) {
+    e = hipGetDevice(&was);
+    if (e == hipSuccess && was != device)
+      e = hipSetDevice(device);
+    else
+      was = -1;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+  OnDevice(const OnDevice &) = delete;
+  OnDevice &operator=(const OnDevice &) = delete;
+};
+
 struct aih_model {
   sw::Model g;
+  int device = 0;  // current at load: the one that holds the buffers
   uint32_t n = 1;
   int32_t dt = AIH_F32, wdt = AIH_F32;
   std::vector<void *> allocs;
@@ -1332,6 +1351,7 @@ aih_model *aih_model_load_ex(const void *bytes, size_t len, uint32_t n, int32_t 
     }
     if (!m->g.consts.empty()) return api_fail("model_load: constant tensors are not supported");
     validate_geometry(m->g);
+    (void)hipGetDevice(&m->device);
     prepare_weights(m.get(), c);
     find_fusions(m.get());
     alloc_tensors(m.get());
@@ -1440,12 +1460,17 @@ int aih_model_read_output(aih_model *m, const char *name, float *host_nhwc, size
     const size_t want = (size_t)m->n * t.h * t.w * t.c;
     if (count != want) return api_fail("read_output: expected " + std::to_string(want) + " floats");
     const aih_model::View &v = m->views[tid];
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    // a stream under capture cannot be waited for: the wait says so, before
-    // anything is recorded
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    hipError_t e = hipStreamIsCapturing(s, &cap);
-    if (e == hipSuccess && cap != hipStreamCaptureStatusNone) e = hipStreamSynchronize(s);
+    // the copy waits for `stream` and then, on the null stream of the model's
+    // device, for every blocking stream: an infer on another one is read whole,
+    // whatever device is current (a stream under capture cannot be waited for:
+    // the wait says so, before anything is recorded)
+    if (stream) {
+      const hipError_t w = hipStreamSynchronize(static_cast<hipStream_t>(stream));
+      if (w != hipSuccess) return hip_fail("read_output", w);
+    }
+    const OnDevice on(m->device);
+    hipStream_t s = nullptr;
+    hipError_t e = on.e;
     if (e != hipSuccess) return hip_fail("read_output", e);
     // unpacked on the device behind the work that writes the tensor, then
     // copied straight to the caller (one frame of the real segmentation model,

@@ -20,6 +20,7 @@
   through the native loader.
 Outputs of the op tests start as NaN.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -353,6 +354,31 @@ def test_real_model_fp32_every_op_matches_oracle(segm, n, fuse):
     m.upload_input("input_1", torch.from_numpy(x2).cuda())
     m.infer()
     assert G.rel_err(m.read_output(), graph.run({"input_1": x2}, n=n)["segment"]) <= 1e-3
+    m.close()
+
+
+def test_read_output_waits_for_blocking_streams(segm):
+    """read_output through one stream of what another, blocking stream still
+    computes: the copy waits for both (it runs on the null stream)."""
+    data, _ = segm
+    m = sw.SwModel(data, n=8)
+    x = [torch.from_numpy(rnd(65 + i, 8, 160, 288, 3)).cuda() for i in range(2)]
+    want = []
+    for xi in (x[1], x[0]):  # the output holds x[0]'s at the end
+        m.upload_input("input_1", xi)
+        m.infer()
+        want.append(m.read_output())
+    assert not np.array_equal(*want)
+    m.upload_input("input_1", x[1])
+    torch.cuda.synchronize()
+    a = ctypes.c_void_p()
+    assert int(torch.cuda.cudart().cudaStreamCreate(ctypes.addressof(a))) == 0
+    for _ in range(100):  # some 20 ms
+        m.infer(stream=a.value)
+    got = m.read_output(stream=torch.cuda.Stream())
+    torch.cuda.synchronize()
+    assert int(torch.cuda.cudart().cudaStreamDestroy(a.value)) == 0
+    assert np.array_equal(got, want[0])
     m.close()
 
 
