@@ -99,7 +99,7 @@ std::string json_quote(const std::string &s) {
 
 using namespace aih;
 
-constexpr size_t kReadFloats = 16u << 20;
+constexpr size_t kReadFloats = 16u << 20, kReadFloatsMin = 1u << 16;
 
 // Makes `device` current while it lives.
 struct OnDevice {
@@ -140,7 +140,8 @@ struct aih_model {
   float *staging = nullptr;
   size_t staging_floats = 0;
   // read_output's logical fp32 values on their way to the host, an output (or
-  // kReadFloats of a larger tensor) at a time; one reader at a time holds it
+  // kReadFloats of a larger tensor) at a time, from the first read on; one
+  // reader at a time holds it
   float *reading = nullptr;
   size_t read_floats = 0;
   std::mutex read_mutex;
@@ -173,6 +174,7 @@ struct aih_model {
 
   ~aih_model() {
     for (void *p : allocs) (void)hipFree(p);
+    (void)hipFree(reading);
   }
 
   void *dalloc(size_t bytes) {
@@ -182,6 +184,28 @@ struct aih_model {
     allocs.push_back(p);
     device_bytes += bytes;
     return p;
+  }
+
+  // The buffer of read_output: 64 MB at most, and a pixel of any tensor; less
+  // (kReadFloatsMin) where the device has no room for an output.
+  hipError_t alloc_reading() {
+    if (reading) return hipSuccess;
+    size_t pixel = 0, whole = 0;
+    for (const auto &t : g.tensors) pixel = std::max<size_t>(pixel, t.c);
+    for (uint32_t t : g.outputs)
+      whole = std::max(whole, (size_t)n * g.tensors[t].h * g.tensors[t].w * g.tensors[t].c);
+    hipError_t e = hipSuccess;
+    for (size_t f : {std::min(std::max(whole, kReadFloatsMin), kReadFloats), kReadFloatsMin}) {
+      read_floats = std::max(f, pixel);
+      void *p = nullptr;
+      e = hipMalloc(&p, read_floats * 4);
+      if (e == hipSuccess) {
+        reading = static_cast<float *>(p);
+        break;
+      }
+      (void)hipGetLastError();
+    }
+    return e;
   }
 
   int64_t find(const char *name) const {
@@ -1360,12 +1384,6 @@ aih_model *aih_model_load_ex(const void *bytes, size_t len, uint32_t n, int32_t 
     for (uint32_t t : m->g.inputs)
       m->staging_floats = std::max(m->staging_floats, (size_t)n * m->g.tensors[t].h * m->g.tensors[t].w * m->g.tensors[t].c);
     if (m->staging_floats) m->staging = static_cast<float *>(m->dalloc(m->staging_floats * 4));
-    // 64 MB at most, and a pixel of any tensor
-    for (uint32_t t : m->g.outputs)
-      m->read_floats = std::max(m->read_floats, (size_t)n * m->g.tensors[t].h * m->g.tensors[t].w * m->g.tensors[t].c);
-    m->read_floats = std::min(std::max<size_t>(m->read_floats, 1u << 16), kReadFloats);
-    for (const auto &t : m->g.tensors) m->read_floats = std::max<size_t>(m->read_floats, t.c);
-    m->reading = static_cast<float *>(m->dalloc(m->read_floats * 4));
     lower(m.get());
     if (m->ws_bytes) m->ws = m->dalloc(m->ws_bytes);
     fuse_stem_launch(m.get());
@@ -1477,6 +1495,8 @@ int aih_model_read_output(aih_model *m, const char *name, float *host_nhwc, size
     // 160x288x2 fp32, host memory in and out: 331 us a call with the padded
     // copy and the host's pass over it, 300 here)
     std::lock_guard<std::mutex> lock(m->read_mutex);
+    e = m->alloc_reading();
+    if (e != hipSuccess) return hip_fail("read_output", e);
     const size_t px = (size_t)m->n * t.h * t.w, step = m->read_floats / t.c;
     for (size_t p = 0; p < px && e == hipSuccess; p += step) {
       const size_t k = std::min(step, px - p);

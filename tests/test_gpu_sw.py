@@ -357,6 +357,26 @@ def test_real_model_fp32_every_op_matches_oracle(segm, n, fuse):
     m.close()
 
 
+def test_the_copy_buffer_comes_with_the_first_read(segm):
+    """A model whose results are read where they lie holds no buffer for
+    read_output: its device bytes are its weights, tensors, staging and
+    workspace, and the first read alone allocates."""
+    data, _ = segm
+    x = torch.from_numpy(rnd(64, 64, 160, 288, 3)).cuda()
+    m = sw.SwModel(data, n=64)
+    m.upload_input("input_1", x)
+    m.infer()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    buffer = 64 * 160 * 288 * 2 * 4
+    y = m.read_output()
+    held = free - torch.cuda.mem_get_info()[0]
+    assert buffer <= held <= buffer + (4 << 20), held
+    assert np.array_equal(m.read_output(), y)
+    assert torch.cuda.mem_get_info()[0] == free - held
+    m.close()
+
+
 def test_read_output_waits_for_blocking_streams(segm):
     """read_output through one stream of what another, blocking stream still
     computes: the copy waits for both (it runs on the null stream)."""
