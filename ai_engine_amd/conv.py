@@ -241,12 +241,19 @@ def _ptr(t) -> int | None:
     return t.data_ptr()
 
 
+_current = None  # torch's current device and raw current stream
+
+
 def _stream(stream) -> int | None:
     if stream is None:
-        import torch
+        global _current
+        if _current is None:
+            import torch
 
-        # torch.cuda.current_stream().cuda_stream without its Stream object
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+            # torch.cuda.current_stream().cuda_stream without its Stream object
+            _current = torch.cuda.current_device, torch._C._cuda_getCurrentRawStream
+        device, raw = _current
+        return raw(device())
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -261,20 +268,22 @@ def _workspace(nbytes: int, ws, device):
 
 
 def _desc_of(spec, fields):
-    """spec.desc(), built again only when a field's value differs from the last
-    run's (a launch's descriptor takes as long to build as the rest of the
-    call). The values are compared, so a changed spec is never run with an old
-    descriptor; a spec with a field that can change in place (a list), or of a
-    class derived from these, builds it every time. The C side only reads it."""
+    """spec.desc(), built again only when a field's value or type differs from
+    the last run's (a launch's descriptor takes as long to build as the rest of
+    the call). The values are compared, so a changed spec is never run with an
+    old descriptor, and their types, so that what desc() refuses (1.0 for 1) is
+    refused again; a spec with a field that can change in place (a list), or of
+    a class derived from these, builds it every time. The C side only reads it."""
     key = fields(spec)
     last = spec.__dict__.get("_last_desc")
-    if last is not None and last[0] == key:
-        return last[1]
+    if last is not None and last[0] == key and last[1] == [*map(type, key)] and (
+            spec.pad is last[2] or all(type(e) is int for e in spec.pad)):
+        return last[3]
     d = spec.desc()
     if type(spec) in (ConvOp, IrBlockSpec, DwPwSpec) and all(
             type(v) in _PLAIN or isinstance(v, enum.IntEnum) or
             (type(v) is tuple and all(type(e) is int for e in v)) for v in key):
-        spec.__dict__["_last_desc"] = (key, d)
+        spec.__dict__["_last_desc"] = (key, [*map(type, key)], spec.pad, d)
     return d
 
 

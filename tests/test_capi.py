@@ -4,6 +4,8 @@ oracle's restatement of ai-core pack.rs byte for byte, the variant policy
 behaves as specified, and invalid descriptors fail with -1 and a message
 instead of crashing (the reference FFI's contract, crates/ai-ffi/src/lib.rs:45-52)."""
 import ctypes as C
+import dataclasses
+import enum
 import os
 import re
 
@@ -595,3 +597,71 @@ def test_noalloc_rejects_workspace_beyond_scratch_on_the_host():
     d = op.desc()
     assert L.aih_conv_noalloc(C.byref(d), None, None, None, None, None, None) == -1
     assert str(need) in conv.last_error() and "scratch" in conv.last_error()
+
+
+# ---------------------------------------------------------------- descriptors kept on a spec
+
+SPECS = [(lambda cls=conv.ConvOp: cls(ih=8, iw=9, cin=8, cout=16, kh=3, kw=3, pad=(1, 1, 1, 1)), conv._CONV_FIELDS),
+         (lambda cls=conv.IrBlockSpec: cls(ih=8, iw=9, cin=16, cexp=64, cout=16), conv._IR_FIELDS),
+         (lambda cls=conv.DwPwSpec: cls(ih=8, iw=9, c=16, cout=16), conv._DWPW_FIELDS)]
+
+
+@pytest.mark.parametrize("make,fields", SPECS, ids=["conv", "block", "dwpw"])
+def test_kept_descriptor_follows_every_field(make, fields):
+    """The descriptor that run() keeps on a spec is that of the spec's present
+    fields: each of them changed in turn, between two runs' descriptors."""
+    def same(spec):
+        return bytes(conv._desc_of(spec, fields)) == bytes(spec.desc())
+
+    for f in dataclasses.fields(make()):
+        spec = make()
+        assert same(spec) and conv._desc_of(spec, fields) is conv._desc_of(spec, fields)
+        old, v = bytes(spec.desc()), getattr(spec, f.name)
+        if isinstance(v, conv.DType) or f.name == "wdt":
+            new = conv.DType.F16
+        elif isinstance(v, conv.Activation):
+            new = conv.Activation.HARDSWISH
+        elif isinstance(v, tuple):
+            new = tuple(e + 1 for e in v)
+        elif isinstance(v, bool):
+            new = not v
+        elif isinstance(v, enum.IntEnum):
+            new = type(v)(2)
+        else:
+            new = 1 + (v or 0)
+        setattr(spec, f.name, new)
+        assert same(spec), f.name
+        assert bytes(conv._desc_of(spec, fields)) != old, f.name
+        setattr(spec, f.name, v)
+        assert bytes(conv._desc_of(spec, fields)) == old, f.name
+    # a list is compared by what it holds now
+    spec = make()
+    spec.pad = [1, 1, 1, 1]
+    assert same(spec)
+    spec.pad[2] = 2
+    assert same(spec) and list(conv._desc_of(spec, fields).pad) == [1, 1, 2, 1]
+    # a derived class may compute its descriptor from more than its fields
+    class Twice(type(make())):
+        k2 = 1
+
+        def desc(self):
+            d = super().desc()
+            d.n *= self.k2
+            return d
+
+    spec = make(Twice)
+    assert conv._desc_of(spec, fields).n == 1
+    spec.k2 = 2
+    assert conv._desc_of(spec, fields).n == 2
+
+
+@pytest.mark.parametrize("make,fields", SPECS, ids=["conv", "block", "dwpw"])
+def test_kept_descriptor_refuses_what_desc_refuses(make, fields):
+    """A value that compares equal to a kept descriptor's but that desc()
+    refuses (1.0 for 1) is refused after a run too."""
+    for name, bad in (("n", 1.0), ("ih", 8.0), ("pad", (1.0, 1, 1, 1))):
+        spec = make()
+        conv._desc_of(spec, fields)
+        setattr(spec, name, bad)
+        with pytest.raises(TypeError):
+            conv._desc_of(spec, fields)
