@@ -283,10 +283,12 @@ __global__ __launch_bounds__(64 * WM * WN) void conv_stream_kernel(ConvStreamArg
     const uint32_t later = nst - 1 - s < (uint32_t)(NST - 2) ? nst - 1 - s : (uint32_t)(NST - 2);
     cs_wait_vm_n<(AI + WI) * (NST - 2)>(later * nmine);
     // every wavefront's copies of stage s are in LDS, and every wavefront is
-    // done with stage s - 1, whose buffer the next request reuses (its LDS
-    // reads returned before its MFMAs). A bare barrier: __syncthreads()'s
-    // workgroup fence would also wait for the copies still in flight.
-    __asm__ volatile("s_barrier" ::: "memory");
+    // done with stage s - 1, whose buffer the next request reuses: its LDS
+    // reads have returned (written out, so that it does not hang on where the
+    // compiler puts the MFMAs that wait for them). A bare barrier:
+    // __syncthreads()'s workgroup fence would also wait for the copies still
+    // in flight.
+    __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (s + NST - 1 < nst) issue(b_iss);
     compute(b_cmp);
     b_cmp = b_cmp + 1 == NST ? 0 : b_cmp + 1;
