@@ -214,12 +214,11 @@ enum { PW_TILED = 0, PW_ROWS = 1, PW_DIRECT = 2, PW_LDS = 3, PW_SPLITK = 4, PW_S
 // fp32, beyond 64 in groups of 64, one group per work item), a kg count in whole 16-byte
 // units, 4 to 32 MFMA steps (32-256 fp32 / 64-512 16-bit channels), weights
 // within LDS, and enough 32-pixel blocks (>= 2048) that the launch fills every
-// CU without splitting K.
+// CU without splitting K. Only fp32 calls launch it: the LDS-streamed GEMM
+// takes every 16-bit one (pw_dma_plan), and the route's plan stays.
 bool pw_lds_plan(const aih_pw_desc *d, aih::IgDirectArgs *a) {
   const uint32_t ku = d->dt == AIH_F32 ? 1 : 2, es = d->dt == AIH_F32 ? 4 : 2;
   const uint64_t M = (uint64_t)d->n * d->m;
-  // more than 64 outputs only at fp32: at 16 bit the tiled GEMM is as fast
-  // there (64 -> 256 f16 at 40x72 b64: 51.8 us tiled, 53.4 us here)
   if (d->dt != d->wdt || d->ng < 2 || d->ng * 4 > (d->dt == AIH_F32 ? 256u : 64u) || d->kg % ku ||
       M < 2048ull * 32 || M > 0xffffff00ull)
     return false;
@@ -412,7 +411,7 @@ bool pw_dma_plan(const aih_pw_desc *d, int base, aih::ConvStreamArgs *a, aih::Co
   if (d->variant != AIH_VAR_AUTO || pw_splitk_of(d) != 0 || d->dt != d->wdt || d->kg % ku || d->kg / ku < 4)
     return false;
   const uint64_t M = (uint64_t)d->n * d->m, N4 = (uint64_t)d->ng * 4;
-  const uint64_t xb = M * d->kg * 4 * es, wb = (uint64_t)d->kg_pad * N4 * 4 * es;
+  const uint64_t xb = M * d->kg * 4 * es, wb = (uint64_t)d->kg * N4 * 4 * es;  // the rows of weights it reads
   if (M <= aih::kPwSplitkMaxM || xb >= 0x80000000ull || wb >= 0x80000000ull) return false;
   if (base == PW_DIRECT || base == PW_LDS || base == PW_SPLITK) {
     if (d->dt == AIH_F32 || (N4 <= 32 && d->kg < 16)) return false;

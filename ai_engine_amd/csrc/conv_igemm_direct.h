@@ -1,7 +1,7 @@
 // conv_igemm_direct.h -- launch interface of the 3x3 implicit-GEMM conv with
 // at most 64 output channels whose whole weight tensor fits in LDS (the
 // activations go from memory straight into MFMA operand registers), also
-// launched with one tap for pointwise convs with mid-size K.
+// launched with one tap for fp32 pointwise convs with mid-size K.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,7 +41,7 @@ constexpr uint32_t kIgDirectThreads = 512;
 // half (80 fp32 / 160 16-bit input channels).
 constexpr uint32_t kIgDirectMaxSteps = 10;
 
-// Step counts of the pointwise (1x1) instantiations: a call runs the
+// Step counts of the pointwise (1x1, fp32) instantiations: a call runs the
 // smallest one that holds its steps (the extra steps read zero weights and
 // activations).
 constexpr uint32_t kPwLdsSteps[5] = {8, 12, 16, 24, 32};

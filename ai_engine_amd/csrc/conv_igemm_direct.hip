@@ -1,5 +1,5 @@
 // conv_igemm_direct.hip -- 3x3 implicit-GEMM conv with at most 64 output
-// channels (and, as a one-tap launch, pointwise convs with mid-size K), the
+// channels (and, as a one-tap launch, fp32 pointwise convs with mid-size K), the
 // weights resident in LDS and the activations loaded straight into MFMA
 // operand registers.
 //
@@ -333,15 +333,19 @@ hipError_t launch_nob(const IgDirectArgs &a, hipStream_t st) {
   // operand ring depth D (a divisor of 9 * NJ): 6 / 9 / 12 steps, measured
   // against 3 and 18 on the 16 -> 32 and 32 -> 32 / 64 shapes
   if (PW_ONLY || a.taps == 1) {
-    // 1x1: the steps run up to the instantiation's count (ring 8 / 12 deep)
-    switch (pw_lds_steps(a.nj)) {
-      case 8: return launch_inst<DT, NOB, 1, 8, 8>(a, st);
-      case 12: return launch_inst<DT, NOB, 1, 12, 12>(a, st);
-      case 16: return launch_inst<DT, NOB, 1, 16, 8>(a, st);
-      case 24: return launch_inst<DT, NOB, 1, 24, 12>(a, st);
-      case 32: return launch_inst<DT, NOB, 1, 32, 8>(a, st);
-      default: return hipErrorInvalidValue;
+    // 1x1, fp32 only: the steps run up to the instantiation's count (ring 8 /
+    // 12 deep)
+    if constexpr (DT == DT_F32) {
+      switch (pw_lds_steps(a.nj)) {
+        case 8: return launch_inst<DT, NOB, 1, 8, 8>(a, st);
+        case 12: return launch_inst<DT, NOB, 1, 12, 12>(a, st);
+        case 16: return launch_inst<DT, NOB, 1, 16, 8>(a, st);
+        case 24: return launch_inst<DT, NOB, 1, 24, 12>(a, st);
+        case 32: return launch_inst<DT, NOB, 1, 32, 8>(a, st);
+        default: break;
+      }
     }
+    return hipErrorInvalidValue;
   }
   if constexpr (PW_ONLY) return hipErrorInvalidValue;
   switch (a.nj) {

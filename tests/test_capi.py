@@ -508,6 +508,18 @@ def test_plans_report_the_kernel_that_runs():
     assert ig(D.F16, ih=40, iw=40, cout=256, cin=256, k=7, pad=(3,) * 4)[2] == 64  # 100
 
 
+def test_16bit_one_tap_route_is_streamed():
+    """Every 16-bit call of the one-tap route (mid-size K, at most 64 outputs,
+    2048 blocks of 32 pixels) runs on the LDS-streamed GEMM: its one-tap
+    launch exists at fp32 only. Weights padded far beyond the rows in use too."""
+    for dt in (conv.DType.F16, conv.DType.BF16):
+        for kg in range(34, 129, 2):
+            for ng in (2, 5, 8, 9, 16):
+                for pad in (-(-kg // 4) * 4, 1 << 22):
+                    p = conv.GemmPwSpec(m=65537, kg=kg, ng=ng, dt=dt, kg_pad=pad).plan()
+                    assert (p.variant, p.grid, p.ws_bytes) == (conv.Variant.DIRECT, 1025, 0), (kg, ng, pad, p)
+
+
 def test_ir_block_forced_weight_placement():
     base = dict(ih=40, iw=72, cin=64, cexp=256, cout=64, s=1, n=64, dt=conv.DType.F16)
     for tile in [(0, 0), (8, 8), (4, 16)]:
