@@ -77,6 +77,9 @@ ROUTES = {
     "igemm_stem": (lambda a, dt, s: G.run_igemm(12, 20, 3, 32, 3, 2, (1, 1, 1, 1), a, False, dt, s,
                                                 refs=False), V.DIRECT),
     "dw": (lambda a, dt, s: G.run_dw(12, 20, 32, 3, 1, a, False, dt, s, refs=False), None),
+    # few pixels run "igemm_direct" above with K split over wavefronts; these the direct kernel
+    "igemm_direct_32px": (lambda a, dt, s: G.run_igemm(128, 66, 16, 32, 3, 1, (1, 1, 1, 1), a, False, dt, s,
+                                                       refs=False), V.DIRECT),
 }
 
 
