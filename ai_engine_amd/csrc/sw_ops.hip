@@ -129,9 +129,12 @@ __device__ __forceinline__ void resize_vec(const PartArg &pa, bool resized, uint
 
 // One thread per vec4 of the row pair: rows of up to 1024 vec4s in one
 // workgroup (rounded up to whole wavefronts), longer ones in `bpr` workgroups of
-// about 512. (A thread's loads wait for its index arithmetic and the part's
+// about 256. (A thread's loads wait for its index arithmetic and the part's
 // branch, so threads that stride over a long row wait once per turn: with 256
-// of them 80x144x44 from 40x72x32 + 12 took 12.4 us fp32 b1, here 4.0.)
+// of them 80x144x44 from 40x72x32 + 12 took 12.4 us fp32 b1, here 4.0. Over rows
+// of 1032 to 3000 vec4s, upscales and downscales, fp32 and f16, against them at
+// batch 64 / 16 / 4: workgroups of 256 0.93 / 0.75 / 0.53 of the time, of 512
+// 0.95 / 0.75 / 0.54 with single calls up to 1.11, of 1024 1.00 / 0.78 / 0.55.)
 template <int DT, bool O32>
 __global__ __launch_bounds__(1024) void resize_kernel(Parts parts, uint32_t ih, uint32_t iw, uint32_t oh,
                                                       uint32_t ow, float sy, float sx, int mode, uint32_t cg_out,
@@ -342,7 +345,7 @@ int launch_resize(const char *what, uint32_t n, uint32_t ih, uint32_t iw, uint32
   const uint64_t total = rows * ow * cg;
   if (total > 0xffffff00ull || rows > 0x7fffffffull) return api_fail(w + ": output too large");
   const uint32_t nrow = ow * cg;
-  const uint32_t bpr = nrow <= 1024 ? 1u : (nrow + 511) / 512;
+  const uint32_t bpr = nrow <= 1024 ? 1u : (nrow + 255) / 256;
   const uint32_t threads = ((nrow + bpr - 1) / bpr + 63) / 64 * 64;
   // every part's vec4s (its ih x iw or oh x ow pixels times stride_c / 4) below 4 GiB
   bool o32 = true;

@@ -72,7 +72,9 @@ def rdt(x, dt):
 
 RESIZE_CASES = [(10, 18, 20, 36, "half_pixel"), (40, 72, 80, 144, "half_pixel"), (7, 9, 3, 4, "half_pixel"),
                 (5, 6, 10, 12, "asymmetric"), (80, 144, 160, 288, "half_pixel"), (3, 7, 10, 11, "half_pixel"),
-                (9, 5, 4, 13, "asymmetric")]
+                (9, 5, 4, 13, "asymmetric"),
+                # rows of 1028 and 1280 vec4s: five workgroups, the last ragged or whole
+                (9, 100, 18, 257, "half_pixel"), (5, 64, 9, 320, "asymmetric")]
 
 
 @pytest.mark.parametrize("dt", [F32, F16, BF16], ids=["f32", "f16", "bf16"])
