@@ -293,7 +293,7 @@ bool pw_stream_plan(const aih_pw_desc *d, aih::PwStreamArgs *a, aih::PwStreamSha
 // The LDS-streamed conv GEMM's tile for M pixels x N4 outputs (conv_stream.hip)
 // and the arguments that depend on it. More than 64 outputs: the wide tile
 // that pads the columns least, 64- and 96-column tiles counted at 5/4 of
-// their columns at 16 bit, where the LDS reads per MFMA bound them (320 ->
+// their columns at 16 bit, where a wavefront has fewer MFMAs per LDS read (320 ->
 // 576 bf16 at 40x72 b64: 128 us at 128 columns, 64 of them padding, 153 at
 // 64, 158 at 96; fp32 3x3 64 -> 128 b32: 117 and 121). Up to 64 outputs, and
 // where the wide tiles are fewer than two per CU: 64 x 64 (3x3 256 -> 256
@@ -396,7 +396,7 @@ int plan_pw(const aih_pw_desc *d, GemmPlan *g) {
 // (conv_stream.hip): AIH_VAR_AUTO without a forced split, the same storage
 // for activations and weights, whole 16-byte units, at least 4 of them,
 // buffers within 32-bit offsets.
-//   16 bit: what the tiled GEMM ran (192 -> 768 at 21x37 b64: 64.5 -> 35 us),
+//   16 bit: what the tiled GEMM ran (192 -> 768 at 21x37 b64: 64.5 -> 39 us),
 //   and what the direct kernels ran with more than 32 outputs or at least 64
 //   channels, beyond 2048 pixels (32 -> 64 at 80x144 b64: 56.7 -> 35 us, 128
 //   -> 32 at 40x72 b64: 19.6 -> 12.6; below both, 32 -> 16 at 40x72 b64: 6.0
@@ -710,7 +710,7 @@ bool ig_direct_plan(const aih_igemm_desc *d, uint32_t oh, uint32_t ow, aih::IgDi
 // call is one of the direct 3x3 kernel's; unsplit: the tiled GEMM keeps K
 // whole.
 //   tiled calls at 16 bit: from 48 tiles of 64 x 64 (128 -> 128 3x3 at 40x72
-//   b32: 69.7 -> 41 us; fewer tiles, 256 -> 256 at 10x18 b4 is 48 of them:
+//   b32: 69.5 -> 39 us; fewer tiles, 256 -> 256 at 10x18 b4 is 48 of them:
 //   18.1 -> 15.8), below 100 of them, where the tiled GEMM splits K in 5 to 8,
 //   up to 72 products of K a tile and with the weights within an XCD's 4 MB L2
 //   (720 pixels, 256 outputs, 48 tiles: K = 3200 22.1 -> 21.6, 6400 33.9 ->

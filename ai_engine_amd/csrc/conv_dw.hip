@@ -23,10 +23,12 @@
 // otherwise all rows' loads are out together, and such a row's weights are
 // zeroed instead -- better for one-pixel strips, whose rows are short, and for
 // fp32, where one row of a strip is enough in flight (measured per strip).
-// Before (a branch around each column's load): f16 3x3 S = 2 80x144 128 ch b32
-// 32.4 -> 18.4 us (118 MB), 5x5 80x144 96 ch b16 48.1 -> 26.6, 5x5 20x36 96 ch
-// b64 19.0 -> 10.8, 3x3 40x72 64 ch b64 18.8 -> 13.2, 10x18 96 ch b1 4.1 ->
-// 3.0; fp32 3x3 S = 2 80x144 96 ch b16 19.8 -> 14.5, 5x5 46.4 -> 35.6.
+// A pass over buffers in turn: f16 3x3 S = 2 80x144 128 ch b32 42.3 us with a
+// branch around each column's load, 26.5 here (118 MB, 4.5 TB/s). On one set of
+// buffers again and again, so partly from the 256 MB cache: that call 32.4 ->
+// 18.4, 5x5 80x144 96 ch b16 48.1 -> 26.6, 5x5 20x36 96 ch b64 19.0 -> 10.8, 3x3
+// 40x72 64 ch b64 18.8 -> 13.2, 10x18 96 ch b1 4.1 -> 3.0; fp32 3x3 S = 2 80x144
+// 96 ch b16 19.8 -> 14.5, 5x5 46.4 -> 35.6.
 //
 // conv_dw_kernel is the general fallback (any k, s, dilation).
 #include "aih_device.h"
@@ -246,8 +248,8 @@ static bool launch_strip_px(const DwArgs &a, hipStream_t st, hipError_t *e) {
 // The strip length, by the threads one-pixel strips would make (t1): longer
 // strips load each input column once for up to K / S of their pixels, one-pixel
 // strips keep a small layer's tap loops short and the chip full. Each line's
-// limits are multiples of the CUs; measured on both sides (us per call, f16
-// unless said, 256 CUs: 256 threads a CU are 64K):
+// limits are multiples of the CUs; measured on both sides (us per call on one
+// set of buffers, f16 unless said, 256 CUs: 256 threads a CU are 64K):
 //   K = 3, S = 2: one pixel at every size (80x144 128 ch b32 18.4, strips of 4
 //     21.7; fp32 80x144 96 ch b16 14.5 / 16.4). Nothing is shared but a border
 //     column.

@@ -1,7 +1,6 @@
 // conv_stream.h -- launch interface of the conv GEMM whose operands stream
 // through LDS by DMA (buffer loads straight into LDS): pointwise and KxK
-// convs over one input (a plain tensor or a channel view) with more outputs
-// than the direct kernels keep resident.
+// convs over one input (a plain tensor or a channel view).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -41,8 +40,9 @@ struct ConvStreamShape {
   uint32_t wm, wn, tm, tn, bku, nst;
 };
 
-// Tiles for grids of at least two per CU, and for smaller ones (the first
-// where a tap has 8 units).
+// Tiles for more than 64 outputs in grids of at least two a CU, and for the
+// rest (the first for long sums: a KxK tap of 8 units or more, a pointwise K
+// of 40).
 constexpr ConvStreamShape kConvStreamWide[] = {
     {2, 2, 2, 2, 4, 2},  // 128 x 128
     {4, 1, 1, 2, 4, 3},  // 128 x 64

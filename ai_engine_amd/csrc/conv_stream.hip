@@ -5,7 +5,7 @@
 // with the bias -> act -> +residual epilogue of common/epilogue.rs:13-30.
 //
 // K is one sequence of 16-byte units (4 fp32 / 8 16-bit channels), tap-major;
-// a stage is 4 units. A stage's pixel rows and weight rows go from memory to
+// a stage is BKU = 4 or 8 units. A stage's pixel rows and weight rows go from memory to
 // LDS without passing through registers, NST - 1 stages ahead of the MFMAs:
 // out-of-image taps, missing pixels, missing columns and the K tail get an
 // offset past the buffer, which the DMA fills with zeros. The implicit
@@ -29,16 +29,20 @@
 // LDS rows (the stage buffers, free by then), so stores and residual loads
 // move whole runs of a pixel's channels, 16 bytes a lane.
 //
-// What bounds it: at 16 bit the LDS. A wavefront's 2 x 2 blocks read 1 KB per
-// 32-cycle MFMA, 128 bytes a cycle over four SIMDs, the whole LDS rate, and
-// the DMA writes come on top; 128 x 128 tiles reach 675 TFLOP/s (3x3 128 ->
-// 128 f16 at 40x72 b32, 69.7 us on the register-staged tiled GEMM, 38 us
-// here; 192 -> 768 f16 at 21x37 b64, HBM-bound at 95 MB, 64.5 -> 37 us). At
-// fp32 the MFMAs do (64 -> 128 3x3 b32: 222 -> 117 us of 86 at the peak).
-// Measured against it on those f16 shapes: 256 x 128 tiles of 8 wavefronts
-// 55 / 41 us and 128 x 192 ones 62 / 43 (fewer workgroups to overlap),
-// stages of 8 units at 128 x 128 49 / 39 (LDS for two workgroups a CU),
-// three stages of 4 42 / 36.
+// What bounds it: at 16 bit the stages' round trips. A 128 x 128 tile's
+// wavefront has 8 MFMAs a stage between two barriers, and of its time 49 %
+// waits, while the MFMAs are busy 26 %, the LDS 29 % and the VALU about 30 %
+// (counters on 3x3 128 -> 128 f16 at 40x72 b32; 192 -> 768 at 21x37 b64: 43 % and
+// 16, 27 and 32 %, 100 MB of HBM traffic at 2.7 TB/s). The LDS rate would come
+// next: 2 x 2 blocks read 1 KB per 32-cycle MFMA, 128 bytes a cycle over four
+// SIMDs. At fp32 the MFMAs bound it (64 -> 128 3x3 b32: busy 63 %, 222 -> 117
+// us of 104 at the rate a large product reaches). Times of a pass over buffers
+// in turn: 3x3 128 -> 128 69.5 us on the register-staged tiled GEMM, 39 here
+// (700 TFLOP/s), 192 -> 768 64.5 and 39. On one set of buffers again and again
+// (38 / 37 us) other shapes of it took: 256 x 128 tiles of 8 wavefronts 55 /
+// 41 and 128 x 192 ones 62 / 43 (fewer workgroups to overlap), stages of 8
+// units at 128 x 128 49 / 39 (LDS for two workgroups a CU), three stages of 4
+// 42 / 36.
 #include <hip/hip_runtime.h>
 
 #include "conv_stream.h"
