@@ -5,8 +5,8 @@
 // gemm_pw_splitk.wgsl:1-57, chosen by gemm_pw.rs:91-102): K cut across the
 // threads of a workgroup and reduced on chip before the epilogue, instead of
 // partial sums through memory and a second launch. (Calls of few such pixels
-// with a short K and many outputs run here too, one wavefront a block: 48 ->
-// 192 at 10x18 fp32 6.4 us on the tiled GEMM, 2.7 here.)
+// with a short K and many outputs run here too, most with one wavefront a
+// block: 48 -> 192 at 10x18 fp32 6.4 us on the tiled GEMM, 2.7 here.)
 //
 // Here a workgroup owns a 16-pixel x 16-channel output block and its W
 // wavefronts split K: wave w runs K steps [w*spw, (w+1)*spw) on MFMA with

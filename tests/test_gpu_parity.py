@@ -129,8 +129,8 @@ PW_DIRECT = [((80, 144, 44, 24), "relu", False, 3501), ((13, 19, 32, 12), "none"
 
 
 # beyond the register-operand kernel (K, or 65-256 outputs in column groups of
-# 64), >= 2048 blocks of 32 pixels: the direct kernel run with one tap
-# (weights in LDS); a ragged last block, steps padded up to the instantiation
+# 64), >= 2048 blocks of 32 pixels: at fp32 the direct kernel run with one tap
+# (weights in LDS), at 16 bit the LDS-streamed GEMM in its place; a ragged last block, steps padded up to the instantiation
 # (25 -> 32, 13 -> 16), a half-empty last step at 16 bit, 4 and 3 column
 # groups (the last one ragged: 136 = 2 x 64 + 8)
 PW_LDS = [((257, 257, 256, 64), "relu", True, 3601), ((260, 256, 200, 20), "hardswish", False, 3602),
@@ -367,7 +367,9 @@ def test_igemm_batch():
 # ---------------------------------------------------------------- the 3x3 direct route (<= 64 outputs)
 
 # (ih, iw, cin or parts, cout, s, d, pad, act, residual, n, seed): every one is
-# routed to the direct kernel in all three dtypes -- odd unit counts per part
+# on the direct route in all three dtypes (with so few pixels the kernel that
+# splits K over wavefronts runs it on a large GPU; the direct kernel itself:
+# tests/test_gpu_igemm_direct.py) -- odd unit counts per part
 # (a half-empty last step), output channels that do not fill a 32-column
 # block, two parts, stride 2, dilation 2, asymmetric padding, residual, a
 # ragged last block of 32 pixels, the largest K per tap
@@ -388,8 +390,7 @@ IG_DIRECT = [
 @pytest.mark.parametrize("case", IG_DIRECT, ids=lambda c: str(c[-1]))
 def test_igemm_direct(case, dt):
     """3x3, cout <= 64, same storage for activations and weights, whole
-    16-byte units per part: the direct route of aih_conv_igemm (weights in
-    LDS, activations straight into MFMA registers)."""
+    16-byte units per part: the direct route of aih_conv_igemm."""
     ih, iw, cin, cout, s, d, pad, act, with_res, n, seed = case
     parts = cin if isinstance(cin, list) else None
     res = G.run_igemm(ih, iw, sum(parts) if parts else cin, cout, 3, s, pad, act, with_res, dt, seed, n=n, d=d,
